@@ -26,13 +26,12 @@
 // row tile), reading each sequence's token range from cu_seqlens on the
 // device.  Prefills of 57 to 64 tokens in all (every sequence one chunk)
 // whose (sequence, v-head) pairs fill at most half the CUs run one launch of
-// the one-chunk kernel: each half-state scan workgroup prepares its
-// sequence's chunk in its own LDS (kernel 2's code) and scans it (kernel
-// 3's), so the slot never goes through the workspace.  Larger prefills run
-// the chunkwise kernels -- after the token kernel's launch, for 2..64
-// sequences that may all be at most 56 tokens long (the host knows only the
-// total): it runs only if every sequence is, and the chunkwise kernels then
-// return at once.
+// the one-chunk kernel: each workgroup prepares its sequence's chunk in its
+// own LDS (kernel 2's code) and scans it (kernel 3's), so the slot never goes
+// through the workspace.  Larger prefills run the chunkwise kernels -- after
+// the token kernel's launch, for 2..64 sequences that may all be at most 56
+// tokens long (the host knows only the total): it runs only if every sequence
+// is, and the chunkwise kernels then return at once.
 //
 // Kernels (one stream, in order):
 //   1. chunk_offsets: one workgroup turns cu_seqlens into the first chunk
@@ -50,13 +49,12 @@
 //      into bf16 hi + lo in the order the scan's MFMAs read them, and the
 //      row scales.
 //   3. scan, one workgroup per (sequence, v-head), XCD-aware order: the
-//      sequential part chunk after chunk with the whole 128 x 128 state in
-//      the registers of eight wavefronts (16 columns each) -- or, for a batch
-//      that would fill at most half the CUs, two workgroups of four
-//      wavefronts per (sequence, v-head), half the state each; the chunk's
-//      K, Q rows and slot reach LDS by DMA a chunk ahead, into the other of
-//      two buffers.  Products with fp32 operands run as bf16 MFMA on hi/lo
-//      splits.  Each workgroup reads its chunks' inputs once, so the
+//      sequential part chunk after chunk.  Four main waves, one a SIMD, hold
+//      the whole 128 x 128 state in registers (32 columns each); four helper
+//      waves beside them bring the next chunk's K, Q rows and slot to LDS by
+//      DMA, into the other of two buffers, and make the K^T and Q K^T tiles
+//      of the current one.  Products with fp32 operands run as bf16 MFMA on
+//      hi/lo splits.  Each workgroup reads its chunks' inputs once, so the
 //      workspace is the only HBM traffic beyond the algorithmic bytes.
 //   One long sequence at few v-heads is cut into segments, since its scan
 //   alone would occupy HV workgroups for the whole run: a first scan launch
@@ -66,20 +64,21 @@
 //   segment starts; a second scan launch runs every segment from its start
 //   with the outputs.
 //
-// MFMA lane layouts (v_mfma_f32_16x16x4_f32, v_mfma_f32_16x16x32_bf16):
-// A[i][k] from lane i + 16 g, B[k][j] from lane j + 16 g (k = g for fp32;
-// for bf16 the lane's 8 items cover the 32-long k block), D[i][j] in lane
-// j + 16 (i / 4), register i % 4.  A bf16 product sums over its k block in
-// any order both operands share.  Where the contracted index is a token,
-// item e of lane group g stands for
-//   k = 16 (e / 4) + 4 g + e % 4,
-// so a lane's 8 items are the 4-element runs at k = 4 g and 16 + 4 g, the
-// runs a 16 x 16 MFMA result holds per lane -- results become operands
-// without exchanging data between lanes.  Where it is a key (K and Q rows
-// read from LDS against the state), item e of lane group g is key 8 g + e of
-// the 32-key block: one 16-byte read per operand, and the 8 lanes that the
-// LDS serves together read 8 rows whose 272-byte stride puts them on
-// disjoint banks.  The state's registers hold its keys in that order.
+// MFMA lane layouts.  16 x 16 (v_mfma_f32_16x16x4_f32, _16x16x32_bf16):
+// A[i][k] from lane i + 16 g, B[k][j] from lane j + 16 g (k = g for fp32; for
+// bf16 the lane's 8 items cover the 32-long k block), D[i][j] in lane j + 16
+// (i / 4), register i % 4.  32 x 32 (_32x32x16_bf16): A[i][k] from lane i +
+// 32 g, B[k][j] from lane j + 32 g (8 items of the 16-long k block), D row 8 q
+// + 4 g + e, column j in lane j + 32 g, register 4 q + e.  A bf16 product sums
+// over its k block in any order both operands share.  Where the contracted
+// index is a token, item e of lane group g of a 16-long block stands for
+//   k = 8 (e / 4) + 4 g + e % 4,
+// so a lane's 8 items are the 4-element runs at k = 4 g and 8 + 4 g, the runs
+// a 32 x 32 result holds per lane -- results become operands without
+// exchanging data between lanes.  Where it is a key (K and Q rows read from
+// LDS against the state), item e of lane group g is key 8 g + e of the block:
+// one 16-byte read per operand.  The state's registers hold its keys in that
+// order.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -93,6 +92,7 @@
 namespace gdn_pf {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -157,39 +157,36 @@ inline bool prep_split(long long slots, int HV) {
   return slots * HV <= kPrepSplitMaxWorkgroups;
 }
 constexpr float kSoftplusThreshold = 20.0f;
-constexpr float kLn2 = 0.693147180559945309f;
+constexpr float kLog2e = 1.44269504088896341f;
 
 // Workspace slot of one (chunk, v-head), offsets in floats.  The scan's MFMA
-// operand T diag(beta) is stored in operand order: a 16 x 32 block is 64
-// lanes x 8 bf16 contiguous (lane = row + 16 g, items in the k order above),
+// operand T diag(beta) is stored in operand order: a 32 x 16 block is 64
+// lanes x 8 bf16 contiguous (lane = row + 32 g, items in the k order above),
 // so a wave reads one with a single 1 KiB access.  It is lower triangular
-// 64 x 64, so only the blocks (row block rb, token block kb) with kb <= rb / 2
-// are kept, six of eight, split into a bf16 high and low part (x ~ hi + lo
+// 64 x 64, so only the blocks (row block rb, token block kb) with kb < 2 rb +
+// 2 are kept, six of eight, split into a bf16 high and low part (x ~ hi + lo
 // to ~2^-16 relative).  Then rows of 64 per-token scales.
-constexpr int kBlk = 512;                             // bf16 per 16 x 32 operand block
+constexpr int kBlk = 512;                             // bf16 per operand block
 constexpr int kBlkF = kBlk / 2;                       // the same in floats
 constexpr int kTriBlocks = 6;
-__host__ __device__ constexpr int tri_blk(int rb, int kb) { return (rb < 3 ? rb : 4) + kb; }
-constexpr int kSlotTh = 0;                            // T diag(beta), hi
-constexpr int kSlotTl = kSlotTh + kTriBlocks * kBlkF; //   lo
-constexpr int kSlotXg = kSlotTl + kTriBlocks * kBlkF; // rk_i e^gamma_i [64]
-constexpr int kSlotEg = kSlotXg + kChunk;             // e^gamma_i [64]
-constexpr int kSlotKs = kSlotEg + kChunk;             // rk_i e^(gamma_C - gamma_i) [64]
-constexpr int kSlotGl = kSlotKs + kChunk;             // e^gamma_C [64 copies]
-constexpr int kSlotGa = kSlotGl + kChunk;             // gamma_i [64]
-constexpr int kSlotRk = kSlotGa + kChunk;             // rk_i [64]
-constexpr int kSlotFloats = kSlotRk + 3 * kChunk;     // padded to whole 1 KiB DMA pieces
-static_assert(kSlotFloats % 256 == 0, "slots stay 1 KiB aligned");
-static_assert(tri_blk(3, 1) == kTriBlocks - 1, "six lower blocks");
+__host__ __device__ constexpr int tri_blk(int rb, int kb) { return 2 * rb + kb; }
+constexpr int kSlotScales = 2 * kTriBlocks * kBlkF;   // after T diag(beta), hi then lo
+// rows of the scales
+constexpr int kRowXg = 0;                             // rk_i e^gamma_i [64]
+constexpr int kRowEg = kRowXg + kChunk;               // scale e^gamma_i [64]
+constexpr int kRowKs = kRowEg + kChunk;               // rk_i e^(gamma_C - gamma_i) [64]
+constexpr int kRowGl = kRowKs + kChunk;               // e^gamma_C [64 copies]
+constexpr int kRowGa = kRowGl + kChunk;               // gamma_i log2(e) [64]
+constexpr int kRowRk = kRowGa + kChunk;               // scale rk_i [64]
+constexpr int kScaleFloats = kRowRk + 3 * kChunk;     // padded to whole 1 KiB DMA pieces
+constexpr int kSlotFloats = kSlotScales + kScaleFloats;
+static_assert(kSlotScales % 256 == 0 && kScaleFloats % 256 == 0, "whole 1 KiB DMA pieces");
+static_assert(tri_blk(1, 3) == kTriBlocks - 1, "six lower blocks");
 
-// Token (0..31) of item e of lane group g inside a 32-long block of a
-// token-contracted operand.
-__host__ __device__ constexpr int k_of(int g, int e) { return 16 * (e >> 2) + 4 * g + (e & 3); }
-
-// First of the 4 keys that register t of a state column holds in lane group
-// g (items e = 0..3 are that key + e): st[2 kb] and st[2 kb + 1] together
-// are keys 32 kb + 8 g .. + 7, the key order of frag().  A 16-row key tile
-// t of the state update is thus keys state_key(t, i / 4) + i % 4.
+// The combine's key order: first of the 4 keys that row tile t holds in lane
+// group g (items e = 0..3 are that key + e): tiles 2 kb and 2 kb + 1 together
+// are keys 32 kb + 8 g .. + 7, the key order of frag().  Row i of tile t is
+// thus key state_key(t, i / 4) + i % 4.
 __host__ __device__ constexpr int state_key(int t, int g) {
   return 32 * (t >> 1) + 8 * g + 4 * (t & 1);
 }
@@ -247,6 +244,11 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
 }
 __device__ __forceinline__ f32x4 mfma_bf16(s16x8 a, s16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                 __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+__device__ __forceinline__ f32x16 mfma32_bf16(s16x8 a, s16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
@@ -313,6 +315,11 @@ __device__ __forceinline__ void seq_range(const Params& p, int s, int& start, in
   start = s0;
   end = s1;
 }
+
+// A value the caller knows is the same in every lane, in a scalar register
+// (the compiler loads what it cannot tell is constant into vector registers,
+// and addresses formed from it stay there).
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // Whether every sequence of a batch of at most 64 has at most `limit`
 // tokens (one read per lane, the clamping of seq_range; uniform).
@@ -484,20 +491,21 @@ __global__ __launch_bounds__(kThreads) void chunk_offsets_kernel(Params p, int32
     slot_info[c] = i32x4{0, 0, 0, 0};
 }
 
-// Gates of token t, v-head hv: log-space decay and beta
-// (g = exp(-exp(A_log) softplus(a + dt_bias)), beta = sigmoid(b)).
+// Gates of token t, v-head hv: the decay's log2 and beta
+// (g = exp(-exp(A_log) softplus(a + dt_bias)), beta = sigmoid(b)).  The decays
+// stay in log2 units: each later exponential is one v_exp_f32.
 __device__ __forceinline__ void gates_of(uint16_t a_raw, uint16_t b_raw, float dt_bias,
-                                         float A_log, float& logg, float& beta) {
+                                         float A_log, float& log2g, float& beta) {
   const float x = bf16_to_f32(a_raw) + dt_bias;
-  const float sp = x > kSoftplusThreshold ? x : __builtin_amdgcn_logf(1.0f + __expf(x)) * kLn2;
-  logg = -__expf(A_log) * sp;
+  const float sp = x > kSoftplusThreshold ? x * kLog2e : __builtin_amdgcn_logf(1.0f + __expf(x));
+  log2g = -__expf(A_log) * sp;
   beta = __builtin_amdgcn_rcpf(1.0f + __expf(-bf16_to_f32(b_raw)));
 }
 
-__device__ __forceinline__ void token_gates(const Params& p, int t, int hv, float& logg,
+__device__ __forceinline__ void token_gates(const Params& p, int t, int hv, float& log2g,
                                             float& beta) {
   gates_of(p.a[static_cast<size_t>(t) * p.HV + hv], p.b[static_cast<size_t>(t) * p.HV + hv],
-           p.dt_bias[hv], p.A_log[hv], logg, beta);
+           p.dt_bias[hv], p.A_log[hv], log2g, beta);
 }
 
 // One DPP step of a wave scan: x from the lane CTRL names (0 where it names
@@ -591,10 +599,11 @@ __device__ __forceinline__ void store16(float* D, int ldd, const f32x4& v, float
 // One chunk's preparation, tokens t0 .. t0 + n - 1 (n: 1..64) of q/k head h,
 // for v-heads hv0 .. hv0 + prep_heads - 1, by the 256 threads of the calling
 // workgroup: the slots go to the workspace (slot c), or with LDS_SLOT (one
-// v-head) to lds_slot in the calling workgroup's LDS.
+// v-head) to lds_T and lds_scales in the calling workgroup's LDS.
 template <bool LDS_SLOT>
 __device__ __forceinline__ void prep_chunk(Params p, int c, int t0, int n, int hv0, int h,
-                                           int prep_heads, PrepLds& lds, float* lds_slot) {
+                                           int prep_heads, PrepLds& lds, uint16_t* lds_T,
+                                           float* lds_scales) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int col = lane & 15;
@@ -674,25 +683,26 @@ __device__ __forceinline__ void prep_chunk(Params p, int c, int t0, int n, int h
   // is rewritten only after the barrier that ends its use.
   for (int j = 0; j < prep_heads; ++j) {
     const int hv = hv0 + j;
-    float* slot = LDS_SLOT ? lds_slot
-                           : p.slots + (static_cast<size_t>(c) * p.HV + hv) * kSlotFloats;
-    uint16_t* slot16 = reinterpret_cast<uint16_t*>(slot);
+    float* const slot = LDS_SLOT ? nullptr
+                                 : p.slots + (static_cast<size_t>(c) * p.HV + hv) * kSlotFloats;
+    uint16_t* const T16 = LDS_SLOT ? lds_T : reinterpret_cast<uint16_t*>(slot);
+    float* const scales = LDS_SLOT ? lds_scales : slot + kSlotScales;
     // gates of token t0 + lane (padded rows: no decay, no update), and the
     // inclusive scan of the log-decay over the chunk
     if (wave == 0) {
-      float logg, beta;
+      float log2g, beta;
       if (j < kPrepGateHeads) {
         uint16_t ar = a_raw[0], br = b_raw[0];
         float dt = dtb[0], al = alog[0];
 #pragma unroll
         for (int jj = 1; jj < kPrepGateHeads; ++jj)
           if (j == jj) { ar = a_raw[jj]; br = b_raw[jj]; dt = dtb[jj]; al = alog[jj]; }
-        gates_of(ar, br, dt, al, logg, beta);
+        gates_of(ar, br, dt, al, log2g, beta);
       } else {
-        token_gates(p, t0 + (lane < n ? lane : n - 1), hv, logg, beta);
+        token_gates(p, t0 + (lane < n ? lane : n - 1), hv, log2g, beta);
       }
-      if (lane >= n) logg = beta = 0.0f;
-      lds.gamma[lane] = wave_prefix_sum(logg);
+      if (lane >= n) log2g = beta = 0.0f;
+      lds.gamma[lane] = wave_prefix_sum(log2g);
       lds.beta[lane] = beta;
     }
     block_sync_lds();
@@ -713,7 +723,7 @@ __device__ __forceinline__ void prep_chunk(Params p, int c, int t0, int n, int h
         const float rkj = lds.rk[j];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float dec = __expf(fminf(gi4[e] - gj, 0.0f));
+          const float dec = __builtin_amdgcn_exp2f(fminf(gi4[e] - gj, 0.0f));
           const float x = bri4[e] * rkj * dec * kk[nj][e];
           lds.A[(ia + e) * kF64Stride + j] = j < ia + e ? x : 0.0f;
         }
@@ -789,43 +799,43 @@ __device__ __forceinline__ void prep_chunk(Params p, int c, int t0, int n, int h
     block_sync_lds();
 
     // T diag(beta) in operand order: lower block (rb, kb) holds, for lane
-    // (col, g), T[16 rb + col][32 kb + k] beta[32 kb + k] at the 8 k of its
-    // items.  Wave w writes block w, waves 0 and 1 also blocks 4 and 5.
-    // Blocks (0, 0) and (2, 1) read T_01 and T_23 (zero); none reads the
-    // recursion's scratch quarter.
+    // (m, g), T[32 rb + m][16 kb + k] beta[16 kb + k] at the 8 k of its items
+    // (4 g .. + 3 and 8 + 4 g .. + 3).  Wave w writes block w, waves 0 and 1
+    // also blocks 4 and 5.  Blocks (0, 1) and (1, 3) read T_01 and T_23
+    // (zero); none reads the recursion's scratch quarter.
 #pragma unroll
     for (int rep = 0; rep < 2; ++rep) {
       const int idx = wave + 4 * rep;
       if (idx >= kTriBlocks) break;                  // uniform per wave
-      const int rb = idx < 3 ? idx : (idx + 2) >> 1;     // tri_blk(rb, kb) == idx
-      const int kb = idx == 3 || idx == 5 ? 1 : 0;
-      const float* trow = &lds.T[(16 * rb + col) * kF64Stride + 32 * kb + 4 * g4];
-      const float* brow = &lds.beta[32 * kb + 4 * g4];
+      const int rb = idx < 2 ? 0 : 1, kb = idx - 2 * rb;     // tri_blk(rb, kb) == idx
+      const int g2 = lane >> 5;
+      const float* trow = &lds.T[(32 * rb + (lane & 31)) * kF64Stride + 16 * kb + 4 * g2];
+      const float* brow = &lds.beta[16 * kb + 4 * g2];
       s16x4 hi[2], lo[2];
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf)
-        split4(*reinterpret_cast<const f32x4*>(trow + 16 * hf) *
-                   *reinterpret_cast<const f32x4*>(brow + 16 * hf),
+        split4(*reinterpret_cast<const f32x4*>(trow + 8 * hf) *
+                   *reinterpret_cast<const f32x4*>(brow + 8 * hf),
                hi[hf], lo[hf]);
-      const int bo = idx * kBlk + lane * 8;
-      *reinterpret_cast<s16x8*>(slot16 + 2 * kSlotTh + bo) = cat(hi[0], hi[1]);
-      *reinterpret_cast<s16x8*>(slot16 + 2 * kSlotTl + bo) = cat(lo[0], lo[1]);
+      uint16_t* const dst = T16 + idx * kBlk + lane * 8;
+      *reinterpret_cast<s16x8*>(dst) = cat(hi[0], hi[1]);
+      *reinterpret_cast<s16x8*>(dst + kTriBlocks * kBlk) = cat(lo[0], lo[1]);
     }
 
     // Row scales for the scan: the decayed K rows of X, the decay of the
-    // output's rows, the K rows of the state update, the chunk decay, and
-    // gamma and the K row scales for its P.
+    // output's rows (times the scale), the K rows of the state update, the
+    // chunk decay, and gamma and the K row scales (times the scale) for its P.
     if (wave == 1) {
       const float gl = lds.gamma[kChunk - 1];        // padded rows carry gamma forward
       const float gi = lds.gamma[lane];
       const float rki = lds.rk[lane];
-      const float egi = __expf(gi);
-      slot[kSlotXg + lane] = rki * egi;
-      slot[kSlotEg + lane] = egi;
-      slot[kSlotKs + lane] = rki * __expf(gl - gi);
-      slot[kSlotGl + lane] = __expf(gl);
-      slot[kSlotGa + lane] = gi;
-      slot[kSlotRk + lane] = rki;
+      const float egi = __builtin_amdgcn_exp2f(gi);
+      scales[kRowXg + lane] = rki * egi;
+      scales[kRowEg + lane] = p.scale * egi;
+      scales[kRowKs + lane] = rki * __builtin_amdgcn_exp2f(gl - gi);
+      scales[kRowGl + lane] = __builtin_amdgcn_exp2f(gl);
+      scales[kRowGa + lane] = gi;
+      scales[kRowRk + lane] = p.scale * rki;
     }
     block_sync_lds();                        // this v-head's LDS reads are done
   }
@@ -867,86 +877,94 @@ void prep_kernel(Params p) {
     n = info.z;
   }
   if (n <= 0) return;                              // uniform per workgroup
-  prep_chunk<false>(p, c, t0, n, hv0, h, p.prep_heads, lds, nullptr);
+  prep_chunk<false>(p, c, t0, n, hv0, h, p.prep_heads, lds, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------
-// 3. the scan: one workgroup per (sequence, v-head) and the whole state, or
-//    two per (sequence, v-head) and half the state each
+// 3. the scan: one workgroup per (sequence, v-head) and the whole state
 // ---------------------------------------------------------------------------
-// W waves (8, two per SIMD; or 4, one per SIMD): the wave of column wave w
-// keeps state columns 16 w .. 16 w + 15 of all 128 keys in registers, st[t]
-// holding keys state_key(t, g) + e of column 16 w + col (lane (col, g)).
-// Read as pairs (st[2 kb], st[2 kb + 1]: keys 32 kb + 8 g .. + 7), the same
-// registers are the state's operand of a product over keys in either role
-// (B of K S, A of S^T Q^T), in the key order of the K and Q operands read
-// from LDS, and every per-chunk result is the next product's operand in
-// place.  Per chunk, with S its start state:
+// Four main waves, one per SIMD, and four helper waves, one beside each.
+// Main wave w keeps 32 columns of the state in registers (all 128 keys: st[t]
+// is the 32 x 32 tile of keys 32 t ..); its lane (m, g) = (lane % 32, lane /
+// 32) holds column 32 w + perm32(m), register r of tile t the key 32 t + 16
+// (r / 8) + 8 g + r % 8.  Registers 8 h .. 8 h + 7 of a tile are thus 8
+// consecutive keys: the state's operand of a product over keys in either role
+// (B of K S, A of S^T Q^T) against 16-byte pieces of K and Q rows, and every
+// per-chunk result is the next product's operand in place.  Per chunk, with S
+// its start state:
 //   X      = V - diag(rk e^gamma) K S
 //   Delta  = T diag(beta) X
 //   O^T    = S^T Q^T diag(scale rq e^gamma) + Delta^T P^T
 //   S     <- e^gamma_C S + K^T diag(rk e^(gamma_C - gamma)) Delta
-// as bf16 MFMA (16x16x32): K, Q, V are bf16; S, X, Delta, T diag(beta) and
+// as bf16 MFMA (32x32x16): K, Q, V are bf16; S, X, Delta, T diag(beta) and
 // P enter split into hi + lo, and a product x y is hi_x hi_y + hi_x lo_y +
 // lo_x hi_y (the lo lo term is ~2^-16 relative and dropped).
+//
+// What bounds it is issue: on a SIMD an MFMA takes ~8 cycles of issue
+// whatever its size and a VALU instruction ~4 (measured: two fp32 FMAs a wave
+// fit under a 16x16x32 for free, six under a 32x32x16), and one wave alone
+// issues an instruction every ~5.5 cycles.  So the larger product (half the
+// instructions, half the LDS reads a column of the 16-column waves before
+// it), and everything the chain over the chunks does not need off the main
+// waves: their DMA (~1.7 k cycles a chunk held at the issue), K^T and P' tiles
+// (~2.2 k) and Q norms (~0.4 k) take the helpers' issue slots.  Measured
+// against eight 16-column waves that each did a share of everything, kernel
+// trace: 64 x 512 tokens at 16/32 heads 429-463 -> 365-405 us, 12 ragged
+// sequences of 7-2048 tokens there 191 -> 152 us, 16 x 1024 at 4/8 76
+// (half-state workgroups on twice the CUs) -> 66 us; ~9.4 k cycles a chunk
+// step.  With all CUs at it the clock falls under the MFMA load (64 x 512: 0.87
+// PFLOP/s of bf16 products, where a plain 8192^3 product reaches 1.26).
 //
 // The waves share the chunk's K rows, Q rows and workspace slot, which the
 // LDS DMA (global_load_lds_dwordx4: each lane's 16 bytes land at the wave's
 // LDS base + 16 lane, no registers) brings into one of two LDS buffers while
 // the chunk before runs on the other.  The operands with tokens as the
-// contracted index come from products with a selector (a 32 x 16 block of
-// the identity), which moves a 16 x 32 row block's columns into the result
-// layout exactly: V^T tiles (each wave's own 16 columns of V, loaded into
-// registers a chunk ahead) and K^T tiles (wave w makes key tiles w, w + W,
-// ... from the K rows in LDS and shares them through LDS: a second barrier
-// per chunk, before the state update).
-constexpr int kScanWaves = 8;
-constexpr int kScanThreads = 64 * kScanWaves;
-// A scan workgroup of W waves holds 16 W state columns: W = 8, the whole
-// state, or W = 4, half of it (columns 64 half .. + 63), two workgroups per
-// (sequence, v-head).  A workgroup holds a CU alone (its LDS), so with W = 4
-// each SIMD runs one wave instead of two: a chunk step costs about half
-// (its instruction issue, which the two waves of a SIMD share, sets it), for
-// twice the workgroups -- the form for batches whose whole-state workgroups
-// would fill at most half the CUs.
-constexpr int kRowPieces = kDim / 8 + 1;          // 16-byte pieces per K / Q row, one of padding
-constexpr int kRowStride = kRowPieces * 8;        // bf16 (68 dwords)
-constexpr int kRowDma = kChunk * kRowPieces / 64; // DMA instructions per K / Q chunk (17)
-constexpr int kSlotDma = kSlotFloats / 4 / 64;    // DMA instructions per slot (14)
-static_assert(kChunk * kRowPieces % 64 == 0 && kSlotFloats % 256 == 0, "whole DMA instructions");
+// contracted index come from products with a selector (a 32 x 32
+// permutation), which moves a 32 x 32 tile's columns into the result layout
+// exactly: V^T tiles (each main wave's own 32 columns of V, loaded into
+// registers) and K^T tiles (helper w makes key tile w from the K rows in LDS
+// and shares it through LDS).  Two barriers a chunk: the helpers' tiles made
+// and the buffer's last reads before the second half; the next chunk landed.
+constexpr int kScanWaves = 4;
+constexpr int kScanThreads = 2 * 64 * kScanWaves;
+static_assert(64 * kScanWaves == kThreads, "the one-chunk kernel: main waves only");
+constexpr int kRowDma = kChunk * kDim / 8 / 64;   // DMA instructions per K / Q chunk (16)
+constexpr int kTriDma = 2 * kTriBlocks * kBlk / 8 / 64;   // T diag(beta), hi and lo (12)
+constexpr int kScaleDma = kScaleFloats / 4 / 64;  // row scales (2)
 // K^T operand blocks of a chunk: (key tile t, token block kb), 64 lanes x 8 bf16
-constexpr int kKtElems = 8 * 2 * 64 * 8;
+constexpr int kKtElems = 4 * 4 * kBlk;
 // P' operand blocks (the six lower (row block, token block) ones), hi then lo
 constexpr int kPElems = 2 * kTriBlocks * kBlk;
 
-// 16-byte aligned: the scan reads its row scales as 16-byte vectors.
-template <bool OUT> struct ScanBuf;
-template <> struct __attribute__((aligned(16))) ScanBuf<true> {
-  uint16_t Kr[kChunk * kRowStride];
-  uint16_t Qr[kChunk * kRowStride];
-  float slot[kSlotFloats];
+// A chunk's K and Q rows (256 bytes each) and T diag(beta).  The 16-byte
+// piece p of row r is at position p ^ (r % 16) of the row: the 8 lanes the
+// LDS serves together read one piece of 8 rows, on disjoint banks.
+template <bool OUT> struct ScanIn;
+template <> struct __attribute__((aligned(16))) ScanIn<true> {
+  uint16_t Kr[kChunk * kDim];
+  uint16_t Qr[kChunk * kDim];
+  uint16_t T[2 * kTriBlocks * kBlk];
 };
-template <> struct __attribute__((aligned(16))) ScanBuf<false> {  // without outputs: no Q
-  uint16_t Kr[kChunk * kRowStride];
-  float slot[kSlotFloats];
+template <> struct __attribute__((aligned(16))) ScanIn<false> {  // without outputs: no Q
+  uint16_t Kr[kChunk * kDim];
+  uint16_t T[2 * kTriBlocks * kBlk];
 };
-static_assert(2 * sizeof(ScanBuf<true>) + 2 * (kKtElems + kPElems) <= 160 * 1024,
+struct __attribute__((aligned(16))) ScanScales {
+  float row[kScaleFloats];
+};
+static_assert(2 * sizeof(ScanIn<true>) + 2 * sizeof(ScanScales) + 2 * (kKtElems + kPElems) +
+                  4 * kChunk + 4 * kBlk <= 160 * 1024,
               "one scan workgroup per CU");
 
 typedef __attribute__((address_space(1))) void global_void;
 typedef __attribute__((address_space(3))) void lds_void;
 
-// One wave's DMA instruction: lane l's 16 bytes from src_l to dst + 16 l
+// One wave's DMA instruction: lane l's 16 bytes from base + byte_off (the
+// base the same for the whole workgroup, in scalar registers) to dst + 16 l
 // (dst the same for the whole wave).
-__device__ __forceinline__ void dma16(const void* src_l, void* dst) {
-  __builtin_amdgcn_global_load_lds((global_void*)src_l, (lds_void*)dst, 16, 0, 0);
-}
-
-// The same from a workgroup-uniform base and a 32-bit byte offset per lane:
-// the address form of the instruction with the base in scalar registers, so
-// no lane forms a 64-bit address.
 __device__ __forceinline__ void dma16_at(const void* base, unsigned byte_off, void* dst) {
-  dma16(static_cast<const char*>(base) + byte_off, dst);
+  __builtin_amdgcn_global_load_lds((global_void*)(static_cast<const char*>(base) + byte_off),
+                                   (lds_void*)dst, 16, 0, 0);
 }
 
 // Byte offset of element `item` of token row `row` (< 64) of a bf16 matrix
@@ -961,9 +979,8 @@ __device__ __forceinline__ unsigned row_bytes(int row, unsigned step, unsigned i
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
 // Workgroup barrier after this wave's LDS reads and writes (s_waitcnt
-// lgkmcnt(0)) but not its DMA: a fence on LDS would wait for the DMA in
-// flight too (it writes LDS), which only the next chunk reads.  The empty
-// asm statements keep the compiler from moving memory accesses across.
+// lgkmcnt(0)) but not its global loads in flight.  The empty asm statements
+// keep the compiler from moving memory accesses across.
 __device__ __forceinline__ void barrier_lds_no_dma() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -971,56 +988,48 @@ __device__ __forceinline__ void barrier_lds_no_dma() {
   asm volatile("" ::: "memory");
 }
 
-// DMA of a chunk's K rows, Q rows (OUT; rows >= n repeat row n - 1; each
-// row's padding piece repeats its last piece) and slot (SLOT) into one LDS
-// buffer; wave w of W issues instructions w, w + W, ....
-template <bool OUT, int W, bool SLOT = true>
-__device__ __forceinline__ void scan_dma(ScanBuf<OUT>& B, const uint16_t* kbase,
-                                         const uint16_t* qbase, unsigned step, int n,
-                                         const float* slot, int wave, int lane) {
-  for (int i = wave; i < kRowDma; i += W) {                 // uniform per wave
-    const int pc = i * 64 + lane;
-    const int r = pc / kRowPieces, c = pc % kRowPieces;
-    const unsigned off = row_bytes(r < n ? r : n - 1, step, (c < 16 ? c : 15) * 8);
-    dma16_at(kbase, off, &B.Kr[i * 512]);
-    if constexpr (OUT) dma16_at(qbase, off, &B.Qr[i * 512]);
-  }
-  if constexpr (SLOT) {
-    for (int i = wave; i < kSlotDma; i += W)
-      dma16_at(slot, static_cast<unsigned>(i * 64 + lane) * 16u, &B.slot[i * 256]);
-  }
-}
-
-// This wave's 16 columns of V for token tile r (lane (col, g): token
-// 16 r + col, columns 16 cw + 4 g .. + 3, cw the wave's column wave; rows
-// >= n repeat row n - 1).
-__device__ __forceinline__ void load_v(u32x2 (&f)[4], const uint16_t* vbase, unsigned step, int n,
-                                       int cw, int col, int g4) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = r * 16 + col;
-    f[r] = *reinterpret_cast<const u32x2*>(
-        reinterpret_cast<const char*>(vbase) + row_bytes(row < n ? row : n - 1, step,
-                                                         cw * 16 + g4 * 4));
-  }
-}
-
-__device__ __forceinline__ s16x8 split_hi_lo(const f32x4& a, const f32x4& b, s16x8& lo) {
-  s16x4 ha, la, hb, lb;
-  split4(a, ha, la);
-  split4(b, hb, lb);
-  lo = cat(la, lb);
-  return cat(ha, hb);
+// Operand label m (0..31) of a 32 x 32 result's row or column as the key (or
+// state column) it stands for: result row 8 q + 4 g + e, register 4 q + e of
+// lane group g, is key 16 (q / 2) + 8 g + 4 (q % 2) + e, so that a lane's
+// registers 8 h .. 8 h + 7 are the keys 16 h + 8 g .. + 7.
+__device__ __forceinline__ int perm32(int m) {
+  return (m & 0x13) | ((m & 4) << 1) | ((m & 8) >> 1);
 }
 
 __device__ __forceinline__ s16x8 ld_op(const void* ptr) {
   return *reinterpret_cast<const s16x8*>(ptr);
 }
 
-// bf16 values held in fp32 back to bf16 (exact), 4 at a time.
-__device__ __forceinline__ s16x4 to_bf16x4(const f32x4& x) {
-  const u32x2 w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
-  return __builtin_bit_cast(s16x4, w);
+// Registers 8 H .. 8 H + 7 of a result tile as hi and lo operand items.
+template <int H>
+__device__ __forceinline__ s16x8 split8(const f32x16& x, s16x8& lo) {
+  s16x4 ha, la, hb, lb;
+  split4(f32x4{x[8 * H], x[8 * H + 1], x[8 * H + 2], x[8 * H + 3]}, ha, la);
+  split4(f32x4{x[8 * H + 4], x[8 * H + 5], x[8 * H + 6], x[8 * H + 7]}, hb, lb);
+  lo = cat(la, lb);
+  return cat(ha, hb);
+}
+
+// Registers 8 H .. 8 H + 7 as bf16 (rounded to nearest even; exact for
+// values that came from bf16).
+template <int H>
+__device__ __forceinline__ s16x8 to_bf16x8(const f32x16& x) {
+  const u32x4 w = {pack_bf16x2(x[8 * H], x[8 * H + 1]), pack_bf16x2(x[8 * H + 2], x[8 * H + 3]),
+                   pack_bf16x2(x[8 * H + 4], x[8 * H + 5]), pack_bf16x2(x[8 * H + 6], x[8 * H + 7])};
+  return __builtin_bit_cast(s16x8, w);
+}
+
+// Four 4-row runs of a result tile's rows (8 q + 4 g, q = 0..3) of a row of
+// per-token scales: token 32 R + 8 q + 4 g + e in item 4 q + e.
+__device__ __forceinline__ f32x16 row_scales(const float* row, int R, int g) {
+  f32x16 s;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(row + 32 * R + 8 * q + 4 * g);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[4 * q + e] = v[e];
+  }
+  return s;
 }
 
 // The per-workgroup constants of a scan.
@@ -1034,31 +1043,8 @@ struct ScanCtx {
   unsigned kstep, vstep;       // elements from one token's K / Q row (V row) to the next
   int start, end, nchunks;     // token range and chunks
   int H, HV, h, hv;
-  float scale;
   bool values;
-  int cw0;                     // the first wave's column wave: 0, or 4 for the second half
 };
-
-// Column wave of wave `wave` (columns 16 cw .. 16 cw + 15): with W = 8 the
-// wave itself (cw0 is 0; known here at compile time).
-template <int W>
-__device__ __forceinline__ int column_wave(const ScanCtx& cx, int wave) {
-  return W == kScanWaves ? wave : cx.cw0 + wave;
-}
-
-// Chunk c's DMA into buf (its slot with SLOT) and its V into registers.
-template <bool OUT, int W, bool SLOT = true>
-__device__ __forceinline__ void scan_issue(ScanBuf<OUT>* buf, const ScanCtx& cx, int c,
-                                           u32x2 (&vf)[4]) {
-  const int wave = wave_index(), lane = threadIdx.x & 63;
-  const int tc = cx.start + c * kChunk;
-  const int nc = min(kChunk, cx.end - tc);
-  scan_dma<OUT, W, SLOT>(*buf, cx.k + (static_cast<size_t>(tc) * cx.H + cx.h) * kDim,
-                   cx.q + (static_cast<size_t>(tc) * cx.H + cx.h) * kDim, cx.kstep, nc,
-                   cx.slot_base + c * cx.slot_step, wave, lane);
-  load_v(vf, cx.v + (static_cast<size_t>(tc) * cx.HV + cx.hv) * kDim, cx.vstep, nc,
-         column_wave<W>(cx, wave), lane & 15, lane >> 4);
-}
 
 // Where chunk c's inputs come from (rows >= n repeat row n - 1).
 struct ChunkSrc {
@@ -1080,435 +1066,478 @@ __device__ __forceinline__ ChunkSrc chunk_src(const ScanCtx& cx, int c) {
   return s;
 }
 
-// Part `part` (0..3) of a chunk's DMA and V loads, so that a chunk step
-// spreads them over its products (issued at once, the eight waves' DMA
-// instructions queue behind each other and hold each wave at the issue for
-// 1-2.5 k cycles): with W = 8, parts 0..2 the K / Q row instructions w + 8
-// part, part 2 also slot instruction w, part 3 slot instruction w + 8 and the
-// V loads; with W = 4 each part issues twice as many, instructions w + 4 j
-// for j = 2 part, 2 part + 1 (rows) and j = 2 (part - 2), 2 (part - 2) + 1
-// (slot).
-template <bool OUT, int W>
-__device__ __forceinline__ void issue_part(ScanBuf<OUT>* __restrict__ Bn, const ScanCtx& cx,
-                                           const ChunkSrc& s, int part, u32x2 (&vf)[4]) {
-  constexpr int kPer = kScanWaves / W;                      // instructions a wave a part
-  const int wave = wave_index(), lane = threadIdx.x & 63;
-  if (part < 3) {
+// Instruction j (0..3) of this wave's share of a K or Q chunk's 16: rows
+// 4 i .. 4 i + 3, i = wave + 4 j, one 16-byte piece a lane (rows >= n repeat
+// row n - 1).
+__device__ __forceinline__ void dma_rows(const uint16_t* base, unsigned step, int n, int j,
+                                         int wave, int lane, uint16_t* dst) {
+  const int i = wave + kScanWaves * j;
+  const unsigned piece = static_cast<unsigned>((lane & 15) ^ (lane >> 4) ^ (4 * (i & 3)));
+  dma16_at(base, row_bytes(min(4 * i + (lane >> 4), n - 1), step, piece * 8), dst + i * 512);
+}
+
+// Part `part` (0..3) of wave `wave`'s (0..3) share of a chunk's DMA into In
+// and Sc (SLOT: its slot too): a K and a Q row instruction, and one of the
+// slot's.
+template <bool OUT, bool SLOT = true>
+__device__ __forceinline__ void issue_part(ScanIn<OUT>* __restrict__ In,
+                                           ScanScales* __restrict__ Sc, const ScanCtx& cx,
+                                           const ChunkSrc& s, int part, int wave, int lane) {
+  dma_rows(s.kbase, cx.kstep, s.n, part, wave, lane, In->Kr);
+  if constexpr (OUT) dma_rows(s.qbase, cx.kstep, s.n, part, wave, lane, In->Qr);
+  if constexpr (SLOT) {
+    static_assert(kTriDma == 3 * kScanWaves && kScaleDma <= kScanWaves, "T in parts 0..2");
+    const int i = wave + kScanWaves * part;
+    const unsigned off = static_cast<unsigned>(lane) * 16u;
+    if (part < 3)
+      dma16_at(s.slot + i * 256, off, In->T + i * 512);
+    else if (wave < kScaleDma)                                // uniform per wave
+      dma16_at(s.slot + i * 256, off, Sc->row + wave * 256);
+  }
+}
+
+// The chunk's V for this wave's 32 columns, as the A operands of the selector products:
+// vf[2 R + b2] is token 32 R + m, columns 32 w + 16 b2 + 8 g .. + 7 (rows
+// >= n repeat row n - 1).
+__device__ __forceinline__ void load_v(u32x4 (&vf)[4], const ScanCtx& cx, const ChunkSrc& s,
+                                       int lane) {
+  const int wave = wave_index();
+  const int m = lane & 31, g = lane >> 5;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = wave + W * (kPer * part + j);
-      if (i < kRowDma) {                                    // uniform per wave
-        const int pc = i * 64 + lane;
-        const int r = pc / kRowPieces, c = pc % kRowPieces;
-        const unsigned off = row_bytes(r < s.n ? r : s.n - 1, cx.kstep, (c < 16 ? c : 15) * 8);
-        dma16_at(s.kbase, off, &Bn->Kr[i * 512]);
-        if constexpr (OUT) dma16_at(s.qbase, off, &Bn->Qr[i * 512]);
+  for (int R = 0; R < 2; ++R) {
+    const int row = 32 * R + m;
+    const unsigned off = row_bytes(min(row, s.n - 1), cx.vstep, 32 * wave + 8 * g);
+#pragma unroll
+    for (int b2 = 0; b2 < 2; ++b2)
+      vf[2 * R + b2] = *reinterpret_cast<const u32x4*>(
+          reinterpret_cast<const char*>(s.vbase) + off + 32 * b2);
+  }
+}
+
+// P' (the B operand blocks of Delta^T P'^T, hi then lo) from the chunk's K
+// and Q rows.  Tile (it, jt): rows i = 16 it + c, tokens j = 16 jt + 4 g4 + e
+// in lane (c, g4) = (lane % 16, lane / 16): items 4 (g4 / 2) + e of lane
+// (i % 32, g4 % 2) of block (it / 2, jt).  Wave w makes tiles w, w + 4 and
+// w + 8 of the ten lower ones and the two above the diagonal inside a block:
+//   it = 0 1 2 3 | 1 3 2 3 | 2 3 0 2, jt = 0 1 2 3 | 0 0 0 1 | 1 2 1 3.
+struct PTile {
+  int it, jt;
+  __device__ __forceinline__ PTile(int wave, int u) {
+    constexpr unsigned kIt = 0x8eede4u, kJt = 0xd940e4u;      // 2 bits a tile
+    it = (kIt >> (2 * (wave + 4 * u))) & 3;
+    jt = (kJt >> (2 * (wave + 4 * u))) & 3;
+  }
+};
+
+// Key block kb's product of a tile: operands from the rows' 16-byte pieces
+// 4 kb + g4 (row r's at position piece ^ (r % 16)).
+__device__ __forceinline__ void p_tile_ops(const uint16_t* Kr, const uint16_t* Qr, PTile pt,
+                                           int kb, int lane, s16x8& ka, s16x8& qb) {
+  const int c = lane & 15, g4 = lane >> 4;
+  const unsigned at = (static_cast<unsigned>(c) * kDim + 8u * (g4 ^ c)) ^ (32u * kb);
+  ka = ld_op(Kr + pt.jt * 16 * kDim + at);
+  qb = ld_op(Qr + pt.it * 16 * kDim + at);
+}
+
+// A finished (K Q^T) tile, scaled and masked, into its blocks.
+__device__ __forceinline__ void p_tile_store(const f32x4& acc, const ScanScales* Sc, PTile pt,
+                                             int lane, uint16_t* Pb) {
+  const int c = lane & 15, g4 = lane >> 4;
+  const float gi = Sc->row[kRowGa + 16 * pt.it + c];
+  const f32x4 gj = *reinterpret_cast<const f32x4*>(&Sc->row[kRowGa + 16 * pt.jt + 4 * g4]);
+  const f32x4 rkj = *reinterpret_cast<const f32x4*>(&Sc->row[kRowRk + 16 * pt.jt + 4 * g4]);
+  const int lim = 16 * (pt.it - pt.jt) + c - 4 * g4;          // j <= i: e <= lim
+  f32x4 pv;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float y = rkj[e] * __builtin_amdgcn_exp2f(fminf(gi - gj[e], 0.0f)) * acc[e];
+    pv[e] = e <= lim ? y : 0.0f;
+  }
+  s16x4 hi, lo;
+  split4(pv, hi, lo);
+  uint16_t* const dst = Pb + tri_blk(pt.it >> 1, pt.jt) * kBlk +
+                        (16 * (pt.it & 1) + c + 32 * (g4 & 1)) * 8 + 4 * (g4 >> 1);
+  *reinterpret_cast<s16x4*>(dst) = hi;
+  *reinterpret_cast<s16x4*>(dst + kTriBlocks * kBlk) = lo;
+}
+
+// What a chunk's second half needs of its K and Q rows, by wave w (0..3) of
+// four: key tile w of K^T (lane (m, g): tokens 32 R + 8 q + 4 g + e of key
+// 32 w + perm32(m), operand blocks (w, 2 R) and (w, 2 R + 1) of Kt), the
+// wave's three P' tiles, and with the L2-norm 1 / |q_i| of Q rows 16 w .. +
+// 15 into Qn.
+template <bool OUT, bool L2>
+__device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
+                                           const ScanScales* __restrict__ Sc,
+                                           uint16_t* __restrict__ Kt, uint16_t* __restrict__ Pb,
+                                           float* __restrict__ Qn,
+                                           const uint16_t* __restrict__ Sel, int w, int lane) {
+  const int m = lane & 31, g = lane >> 5;
+  const unsigned row0 = static_cast<unsigned>(m) * kDim + 8u * (g ^ (m & 15));
+#pragma unroll
+  for (int R = 0; R < 2; ++R) {
+    f32x16 kt;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) kt[r] = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      kt = mfma32_bf16(ld_op(&In->Kr[(row0 ^ (16u * (2 * w + h))) + R * 32 * kDim]),
+                       ld_op(&Sel[h * kBlk + lane * 8]), kt);
+    uint16_t* const dst = Kt + (w * 4 + 2 * R) * kBlk + lane * 8;
+    *reinterpret_cast<s16x8*>(dst) = to_bf16x8<0>(kt);
+    *reinterpret_cast<s16x8*>(dst + kBlk) = to_bf16x8<1>(kt);
+  }
+  if constexpr (OUT) {
+    f32x4 acc[3];
+#pragma unroll
+    for (int u = 0; u < 3; ++u) {
+      acc[u] = f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        s16x8 ka, qb;
+        p_tile_ops(In->Kr, In->Qr, PTile(w, u), kb, lane, ka, qb);
+        acc[u] = mfma_bf16(ka, qb, acc[u]);
       }
     }
-  }
-  if (part >= 2) {
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      const int i = wave + W * (kPer * (part - 2) + j);
-      if (i < kSlotDma)
-        dma16_at(s.slot, static_cast<unsigned>(i * 64 + lane) * 16u, &Bn->slot[i * 256]);
-    }
+    for (int u = 0; u < 3; ++u) p_tile_store(acc[u], Sc, PTile(w, u), lane, Pb);
   }
-  if (part == 3)
-    load_v(vf, s.vbase, cx.vstep, s.n, column_wave<W>(cx, wave), lane & 15, lane >> 4);
+  if constexpr (L2) {
+    // four lanes a row (pieces 4 j + lane % 4: the lanes the LDS serves
+    // together on disjoint banks)
+    const int r = lane >> 2;
+    const uint16_t* const qr = &In->Qr[(16 * w + r) * kDim];
+    float q2 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const u32x4 x = *reinterpret_cast<const u32x4*>(qr + 8 * ((4 * j + (lane & 3)) ^ r));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float lo = __uint_as_float(x[i] << 16);
+        const float hi = __uint_as_float(x[i] & 0xffff0000u);
+        q2 = fmaf(hi, hi, fmaf(lo, lo, q2));
+      }
+    }
+    q2 += __shfl_xor(q2, 1, 64);
+    q2 += __shfl_xor(q2, 2, 64);
+    if ((lane & 3) == 0) Qn[16 * w + r] = __builtin_amdgcn_rsqf(q2 + kL2Eps);
+  }
 }
 
-// P' tiles (row tile r, token tile jt) of a chunk, 10 nonzero and the two
-// zero ones inside the stored blocks (0, 1) and (2, 3); wave w of W makes
-// tiles w, w + W, ....
-// Tile idx is (r, jt) = ((kPTileR >> 2 idx) & 3, (kPTileJ >> 2 idx) & 3):
-//   r  = 0, 1, 1, 2, 2, 2, 3, 3, 3, 3, 0, 2
-//   jt = 0, 0, 1, 0, 1, 2, 0, 1, 2, 3, 1, 3
-// (packed in immediates: a table in memory costs a global load and its wait
-// at the start of every chunk step).
-constexpr int kPTiles = 12;
-constexpr unsigned kPTileR = 0x8ffa94u;
-constexpr unsigned kPTileJ = 0xde4910u;
-
-// Key block kb's product of P' tile IDX, (K Q^T)_(jt, r) over the block,
-// from the K and Q operands of the block's row tiles (in registers).
-template <int IDX>
-__device__ __forceinline__ void p_tile_mma(const s16x8 (&ak)[4], const s16x8 (&bq)[4],
-                                           f32x4& acc) {
-  constexpr int r = (kPTileR >> (2 * IDX)) & 3, jt = (kPTileJ >> (2 * IDX)) & 3;
-  if constexpr (jt <= r) acc = mfma_bf16(ak[jt], bq[r], acc);
+// Chunk ci of a helper wave: the side tiles from In and Sc, then the next
+// chunk's DMA into InN and ScN (their last reads were in the chunk before).
+// All pointers are restrict: the compiler then knows that the DMA never
+// writes what is read meanwhile, and waits for it only at the end.
+template <bool OUT, bool L2>
+__device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
+                                           const ScanScales* __restrict__ Sc,
+                                           ScanIn<OUT>* __restrict__ InN,
+                                           ScanScales* __restrict__ ScN,
+                                           uint16_t* __restrict__ Kt, uint16_t* __restrict__ Pb,
+                                           float* __restrict__ Qn, const ScanCtx& cx,
+                                           const uint16_t* __restrict__ Sel, int ci) {
+  const int lane = threadIdx.x & 63;
+  const int w = wave_index() - kScanWaves;
+  side_tiles<OUT, L2>(In, Sc, Kt, Pb, Qn, Sel, w, lane);
+  if (ci + 1 < cx.nchunks) {                                  // uniform
+    // issued while the main waves finish their first half
+    const ChunkSrc nsrc = chunk_src(cx, ci + 1);
+    issue_part<OUT>(InN, ScN, cx, nsrc, 0, w, lane);
+    issue_part<OUT>(InN, ScN, cx, nsrc, 1, w, lane);
+    barrier_lds_no_dma();
+    issue_part<OUT>(InN, ScN, cx, nsrc, 2, w, lane);
+    issue_part<OUT>(InN, ScN, cx, nsrc, 3, w, lane);
+    wait_vmem();                     // the next chunk's DMA has landed
+  }
+  barrier_lds_no_dma();
 }
 
-// Chunk ci from buffer B, with the next chunk's DMA into Bn; Kt: the K^T
-// operand blocks; Pb: the P' operand blocks (OUT); Qn: the Q row scales
-// (L2).  B, Bn, Kt, Pb and Qn are restrict: the compiler then knows that the
-// DMA in flight into Bn never writes what this chunk reads, and waits for it
-// only at the end.  OUT: the outputs too (else only the state).  L2: the
-// L2-norm (a template flag: as a run-time branch inside the product loop it
-// split the loop into blocks the scheduler could not interleave).
+// Chunk ci of a main wave, from In and Sc (LAST: the last chunk, which may be
+// a partial one); Kt: the K^T operand blocks; Pb: the P' operand blocks
+// (OUT); Qn: the Q row scales (L2).  OUT: the outputs too (else only the
+// state).  L2: the L2-norm.
 //
 // The output's intra-chunk term uses P = diag(rq) P' with
 //   P'_ij = scale rk_j e^(gamma_i - gamma_j) (Q K^T)_ij,  j <= i,
-// made here from the chunk's K and Q rows: (K Q^T) tiles on bf16 MFMA leave
-// each lane 4 consecutive j of one row i, the operand items of P' as the B
-// operand of Delta^T P'^T.  The Q row scales rq = 1 / |q_i| (L2-norm; each
-// wave computes eight rows' from the Q rows in LDS and shares them through
-// Qn) scale the output row: O = diag(rq) (diag(scale e^gamma) Q S + P' Delta).
-template <bool OUT, bool L2, int W, bool FUSE = false>
-__device__ __forceinline__ void scan_chunk(const ScanBuf<OUT>* __restrict__ B,
-                                           ScanBuf<OUT>* __restrict__ Bn,
-                                           uint16_t* __restrict__ Kt, uint16_t* __restrict__ Pb,
-                                           float* __restrict__ Qn, const ScanCtx& cx,
-                                           f32x4 (&st)[8],
-                                           u32x2 (&vnext)[4], const s16x8& sel, int ci) {
-  const int lane = threadIdx.x & 63;
+// made by the helper waves from the chunk's K and Q rows: a (K Q^T) tile on
+// bf16 MFMA (16x16x32) leaves each lane 4 consecutive j of one row i, half
+// the 8 items of a lane of P' as the B operand of Delta^T P'^T.  The Q row
+// scales rq = 1 / |q_i| (L2-norm) scale the output row:
+// O = diag(rq) (diag(scale e^gamma) Q S + P' Delta).
+template <bool OUT, bool L2, bool LAST>
+__device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
+                                           const ScanScales* __restrict__ Sc,
+                                           const uint16_t* __restrict__ Kt,
+                                           const uint16_t* __restrict__ Pb,
+                                           const float* __restrict__ Qn, const ScanCtx& cx,
+                                           f32x16 (&st)[4], const uint16_t* __restrict__ Sel,
+                                           int ci) {
+  // The lane index, opaque to the compiler: it would keep every LDS and
+  // global offset derived from it in a register across the chunks, more than
+  // there are.
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
   const int wave = wave_index();
-  const int col = lane & 15;
-  const int g4 = lane >> 4;
-  const int t0 = cx.start + ci * kChunk;
-  const int n = min(kChunk, cx.end - t0);
-  const int cw = column_wave<W>(cx, wave);   // columns 16 cw .. 16 cw + 15
-  const u32x2 vf[4] = {vnext[0], vnext[1], vnext[2], vnext[3]};
-  // The next chunk's inputs go into the other buffer (after the last chunk:
-  // this one's again, unused) in four parts spread over the K S products.
-  const ChunkSrc nsrc = chunk_src(cx, ci + 1 < cx.nchunks ? ci + 1 : ci);
-  // The chunk's row scales are read where they are used, so that they hold
-  // no registers across the products: B is restrict and 16-byte aligned, so
-  // each read is one ds_read_b128 that the compiler knows the DMA in flight
-  // into Bn does not write (reads it splits into pairs of 4-byte reads lose
-  // that, and wait for the DMA).
+  const int m = lane & 31;
+  const int g = lane >> 5;
 
-  // L2-norm: 1 / |q_i| of Q rows 8 v .. 8 v + 7 into Qn, v = wave + W rep
-  // (lane: row 8 v + lane / 8, items 16 (lane % 8) .. + 15); read after the
-  // barrier below.  (The previous chunk's reads of Qn ended before its last
-  // barrier.)
-  if constexpr (L2) {
-#pragma unroll
-    for (int rep = 0; rep < kScanWaves / W; ++rep) {
-      const int row = 8 * (wave + W * rep) + (lane >> 3);
-      const uint16_t* qr = &B->Qr[row * kRowStride + (lane & 7) * 16];
-      const u32x4 w[2] = {*reinterpret_cast<const u32x4*>(qr),
-                          *reinterpret_cast<const u32x4*>(qr + 8)};
-      float q2 = 0.0f;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float lo = __uint_as_float(w[h][i] << 16);
-          const float hi = __uint_as_float(w[h][i] & 0xffff0000u);
-          q2 = fmaf(hi, hi, fmaf(lo, lo, q2));
-        }
-      q2 += __shfl_xor(q2, 1, 64);
-      q2 += __shfl_xor(q2, 2, 64);
-      q2 += __shfl_xor(q2, 4, 64);
-      if ((lane & 7) == 0) Qn[row] = __builtin_amdgcn_rsqf(q2 + kL2Eps);
-    }
-  }
+  // read ~3 k cycles ahead of their use (a chunk ahead, they hold registers
+  // through the second half, where the most are live)
+  u32x4 vf[4];
+  load_v(vf, cx, chunk_src(cx, ci), lane);
+  __builtin_amdgcn_sched_barrier(0);           // issued here, not before their use
 
-  // K S (token rows) and S^T Q^T (the output's first term, transposed),
-  // one 32-key block of the state at a time.  The K and Q operands of key
-  // block kb + 1 are read into the other of two register sets while block
-  // kb's products run, so the LDS latency is paid once, not per product.
-  // The same operands make this wave's key tiles of K^T (tiles t = wave +
-  // W m, key block t / 2: the selector products of the K row tiles give lane
-  // (col, g) tokens 16 r + 4 g + e of key state_key(t, col / 4) + col % 4)
-  // and its P' tiles' (K Q^T) products, shared with the other waves through
-  // LDS.
-  constexpr int kKtTiles = kScanWaves / W;                  // K^T tiles a wave makes
-  constexpr int kPReps = (kPTiles + W - 1) / W;             // P' tiles a wave makes, at most
-  f32x4 x[4], o[4], pacc[kPReps];
+  // piece 2 b + g of row 32 R + m, at position (2 b + g) ^ (m % 16)
+  const unsigned row0 = static_cast<unsigned>(m) * kDim + 8u * (g ^ (m & 15));
+  auto k_op = [&](int b, int R) { return ld_op(&In->Kr[(row0 ^ (16u * b)) + R * 32 * kDim]); };
+
+  // K S (token rows) and S^T Q^T (the output's first term, transposed), one
+  // 16-key block of the state at a time; block b + 1's operands are read
+  // while block b's products run.
+  f32x16 x[2], o[2];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) x[r] = o[r] = f32x4{0, 0, 0, 0};
+  for (int r = 0; r < 16; ++r) x[0][r] = x[1][r] = o[0][r] = o[1][r] = 0.0f;
+  s16x8 ak[2][2], bq[2][2];
+  auto read_ops = [&](int b, int set) {
 #pragma unroll
-  for (int i = 0; i < kPReps; ++i) pacc[i] = f32x4{0, 0, 0, 0};
-  s16x4 kt[kKtTiles][4];
-  s16x8 ak[2][4], bq[2][4];
-  auto read_ops = [&](int kb, int set) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ak[set][r] = frag(&B->Kr[(r * 16 + col) * kRowStride], kb, g4);
-      if constexpr (OUT) bq[set][r] = frag(&B->Qr[(r * 16 + col) * kRowStride], kb, g4);
+    for (int R = 0; R < 2; ++R) {
+      ak[set][R] = k_op(b, R);
+      if constexpr (OUT) bq[set][R] = ld_op(&In->Qr[(row0 ^ (16u * b)) + R * 32 * kDim]);
     }
   };
   read_ops(0, 0);
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-    const int set = kb & 1;
-    if (kb < 3) read_ops(kb + 1, set ^ 1);
-    if constexpr (!FUSE) issue_part<OUT, W>(Bn, cx, nsrc, kb, vnext);   // FUSE: one chunk
-#pragma unroll
-    for (int m = 0; m < kKtTiles; ++m) {
-      if (kb == ((wave + W * m) >> 1)) {                    // uniform per wave
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          kt[m][r] = to_bf16x4(mfma_bf16(ak[set][r], sel, f32x4{0, 0, 0, 0}));
-      }
-    }
-    if constexpr (OUT && W == 8) {
-      switch (wave) {                                       // uniform per wave
-        case 0: p_tile_mma<0>(ak[set], bq[set], pacc[0]); p_tile_mma<8>(ak[set], bq[set], pacc[1]); break;
-        case 1: p_tile_mma<1>(ak[set], bq[set], pacc[0]); p_tile_mma<9>(ak[set], bq[set], pacc[1]); break;
-        case 2: p_tile_mma<2>(ak[set], bq[set], pacc[0]); break;
-        case 3: p_tile_mma<3>(ak[set], bq[set], pacc[0]); break;
-        case 4: p_tile_mma<4>(ak[set], bq[set], pacc[0]); break;
-        case 5: p_tile_mma<5>(ak[set], bq[set], pacc[0]); break;
-        case 6: p_tile_mma<6>(ak[set], bq[set], pacc[0]); break;
-        default: p_tile_mma<7>(ak[set], bq[set], pacc[0]); break;
-      }
-    } else if constexpr (OUT) {                             // W = 4: tiles w, w + 4, w + 8
-      switch (wave) {                                       // uniform per wave
-        case 0: p_tile_mma<0>(ak[set], bq[set], pacc[0]); p_tile_mma<4>(ak[set], bq[set], pacc[1]);
-                p_tile_mma<8>(ak[set], bq[set], pacc[2]); break;
-        case 1: p_tile_mma<1>(ak[set], bq[set], pacc[0]); p_tile_mma<5>(ak[set], bq[set], pacc[1]);
-                p_tile_mma<9>(ak[set], bq[set], pacc[2]); break;
-        case 2: p_tile_mma<2>(ak[set], bq[set], pacc[0]); p_tile_mma<6>(ak[set], bq[set], pacc[1]);
-                p_tile_mma<10>(ak[set], bq[set], pacc[2]); break;
-        default: p_tile_mma<3>(ak[set], bq[set], pacc[0]); p_tile_mma<7>(ak[set], bq[set], pacc[1]);
-                 p_tile_mma<11>(ak[set], bq[set], pacc[2]); break;
-      }
-    }
+  for (int b = 0; b < 8; ++b) {
+    const int set = b & 1;
+    if (b < 7) read_ops(b + 1, set ^ 1);
     s16x8 sl;
-    const s16x8 sh = split_hi_lo(st[2 * kb], st[2 * kb + 1], sl);
+    const s16x8 sh = (b & 1) ? split8<1>(st[b >> 1], sl) : split8<0>(st[b >> 1], sl);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      x[r] = mfma_bf16(ak[set][r], sh, x[r]);
-      if constexpr (OUT) o[r] = mfma_bf16(sh, bq[set][r], o[r]);
+    for (int R = 0; R < 2; ++R) {
+      x[R] = mfma32_bf16(ak[set][R], sh, x[R]);
+      if constexpr (OUT) o[R] = mfma32_bf16(sh, bq[set][R], o[R]);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      x[r] = mfma_bf16(ak[set][r], sl, x[r]);
-      if constexpr (OUT) o[r] = mfma_bf16(sl, bq[set][r], o[r]);
-    }
-  }
-
-  // this wave's K^T tiles and P' tiles into LDS (read after the barrier below)
-#pragma unroll
-  for (int m = 0; m < kKtTiles; ++m)
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-      *reinterpret_cast<s16x8*>(Kt + (((wave + W * m) * 2 + kb) * 64 + lane) * 8) =
-          cat(kt[m][2 * kb], kt[m][2 * kb + 1]);
-  if constexpr (OUT) {
-    // P' tile (r, jt): lane (col, g) holds row i = 16 r + col, tokens
-    // j = 16 jt + 4 g + e; items 4 (jt % 2) .. + 3 of block (r, jt / 2)
-#pragma unroll
-    for (int rep = 0; rep < kPReps; ++rep) {
-      const int idx = wave + W * rep;
-      if (idx >= kPTiles) break;                       // uniform per wave
-      const int r = (kPTileR >> (2 * idx)) & 3, jt = (kPTileJ >> (2 * idx)) & 3;
-      f32x4 pv = {0, 0, 0, 0};
-      if (jt <= r) {                                   // uniform per wave
-        const int i = r * 16 + col, j0 = jt * 16 + g4 * 4;
-        const float gi = B->slot[kSlotGa + i];
-        const f32x4 gj = *reinterpret_cast<const f32x4*>(&B->slot[kSlotGa + j0]);
-        const f32x4 rkj = *reinterpret_cast<const f32x4*>(&B->slot[kSlotRk + j0]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float x = cx.scale * rkj[e] * __expf(fminf(gi - gj[e], 0.0f)) * pacc[rep][e];
-          pv[e] = j0 + e <= i ? x : 0.0f;
-        }
-      }
-      s16x4 hi, lo;
-      split4(pv, hi, lo);
-      const int at = tri_blk(r, jt >> 1) * kBlk + lane * 8 + (jt & 1) * 4;
-      *reinterpret_cast<s16x4*>(Pb + at) = hi;
-      *reinterpret_cast<s16x4*>(Pb + kTriBlocks * kBlk + at) = lo;
+    for (int R = 0; R < 2; ++R) {
+      x[R] = mfma32_bf16(ak[set][R], sl, x[R]);
+      if constexpr (OUT) o[R] = mfma32_bf16(sl, bq[set][R], o[R]);
     }
   }
 
-  // T diag(beta)'s six lower operand blocks (hi, lo), read while X is formed
-  s16x8 th[kTriBlocks], tl[kTriBlocks];
+  // X = V - diag(rk e^gamma) K S, V^T from the selector products; split
+  s16x8 xh[4], xl[4];
 #pragma unroll
-  for (int b = 0; b < kTriBlocks; ++b) {
-    th[b] = ld_op(&B->slot[kSlotTh + b * kBlkF + lane * 4]);
-    tl[b] = ld_op(&B->slot[kSlotTl + b * kBlkF + lane * 4]);
+  for (int R = 0; R < 2; ++R) {
+    f32x16 v;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = 0.0f;
+    if (cx.values) {                                          // uniform
+      v = mfma32_bf16(__builtin_bit_cast(s16x8, vf[2 * R]), ld_op(&Sel[lane * 8]), v);
+      v = mfma32_bf16(__builtin_bit_cast(s16x8, vf[2 * R + 1]), ld_op(&Sel[kBlk + lane * 8]), v);
+    }
+    const f32x16 xg = row_scales(Sc->row + kRowXg, R, g);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) x[R][r] = v[r] - xg[r] * x[R][r];
+    xh[2 * R] = split8<0>(x[R], xl[2 * R]);
+    xh[2 * R + 1] = split8<1>(x[R], xl[2 * R + 1]);
   }
 
-  // X = V - diag(rk e^gamma) K S: lane (col, g) holds tokens 16 r + 4 g + e
-  // of column 16 cw + col; V^T tiles from the selector products (the
-  // wave's 16 columns sit in the half `cw % 2` = `wave % 2` of a 32-column
-  // block)
+  // Delta = T diag(beta) X (T lower triangular: token blocks kb < 2 R + 2)
+  f32x16 d[2];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const f32x4 xg = *reinterpret_cast<const f32x4*>(&B->slot[kSlotXg + r * 16 + g4 * 4]);
-    const u32x2 vv = cx.values ? vf[r] : u32x2{0u, 0u};
-    const u32x4 w4 = (wave & 1) ? u32x4{0u, 0u, vv.x, vv.y} : u32x4{vv.x, vv.y, 0u, 0u};
-    const f32x4 v = mfma_bf16(__builtin_bit_cast(s16x8, w4), sel, f32x4{0, 0, 0, 0});
-    x[r] = v - xg * x[r];
-  }
-
-  // Delta = T diag(beta) X (T lower triangular: token blocks kb <= r / 2)
-  s16x8 xh[2], xl[2];
+  for (int R = 0; R < 2; ++R) {
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) xh[kb] = split_hi_lo(x[2 * kb], x[2 * kb + 1], xl[kb]);
-  f32x4 d[4];
+    for (int r = 0; r < 16; ++r) d[R][r] = 0.0f;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    d[r] = f32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int kb = 0; kb <= (r >> 1); ++kb) {
-      const int b = tri_blk(r, kb);
-      d[r] = mfma_bf16(th[b], xh[kb], d[r]);
-      d[r] = mfma_bf16(th[b], xl[kb], d[r]);
-      d[r] = mfma_bf16(tl[b], xh[kb], d[r]);
+    for (int kb = 0; kb < 2 * R + 2; ++kb) {
+      const s16x8 th = ld_op(&In->T[tri_blk(R, kb) * kBlk + lane * 8]);
+      const s16x8 tl = ld_op(&In->T[(kTriBlocks + tri_blk(R, kb)) * kBlk + lane * 8]);
+      d[R] = mfma32_bf16(th, xh[kb], d[R]);
+      d[R] = mfma32_bf16(th, xl[kb], d[R]);
+      d[R] = mfma32_bf16(tl, xh[kb], d[R]);
     }
   }
 
   // Delta as operand: A of Delta^T P^T and, scaled by ks, B of the update
-  s16x8 dh[2], dl[2], eh[2], el[2];
-  f32x4 ks[4];
+  s16x8 dh[4], dl[4], eh[4], el[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    ks[r] = *reinterpret_cast<const f32x4*>(&B->slot[kSlotKs + r * 16 + g4 * 4]);
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    if constexpr (OUT) dh[kb] = split_hi_lo(d[2 * kb], d[2 * kb + 1], dl[kb]);
-    eh[kb] = split_hi_lo(d[2 * kb] * ks[2 * kb], d[2 * kb + 1] * ks[2 * kb + 1], el[kb]);
-  }
-
-  // every wave's K^T tile and P' tiles are in LDS past this barrier
-  barrier_lds_no_dma();
-
-  // The operands of the output products two row tiles ahead of their use,
-  // and those of the state update in two halves, the first read with the
-  // output's, the second while the first half's products run.
-  s16x8 ph[kTriBlocks], pl[kTriBlocks], kt_op[8][2];
-  auto read_p = [&](int r) {
-#pragma unroll
-    for (int kb = 0; kb <= (r >> 1); ++kb) {
-      const int b = tri_blk(r, kb);
-      ph[b] = ld_op(Pb + b * kBlk + lane * 8);
-      pl[b] = ld_op(Pb + (kTriBlocks + b) * kBlk + lane * 8);
+  for (int R = 0; R < 2; ++R) {
+    if constexpr (OUT) {
+      dh[2 * R] = split8<0>(d[R], dl[2 * R]);
+      dh[2 * R + 1] = split8<1>(d[R], dl[2 * R + 1]);
     }
-  };
-  if constexpr (OUT) {
-    read_p(0);
-    read_p(1);
+    const f32x16 ks = row_scales(Sc->row + kRowKs, R, g);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) d[R][r] *= ks[r];
+    eh[2 * R] = split8<0>(d[R], el[2 * R]);
+    eh[2 * R + 1] = split8<1>(d[R], el[2 * R + 1]);
   }
-  auto read_kt = [&](int t0k) {
-#pragma unroll
-    for (int t = t0k; t < t0k + 4; ++t)
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) kt_op[t][kb] = ld_op(Kt + ((t * 2 + kb) * 64 + lane) * 8);
-  };
-  read_kt(0);
 
-  // O^T = rq (.) (qs (.) S^T Q^T + Delta^T P'^T); lane (col, g) ends with
-  // columns 16 cw + 4 g + e of token 16 r + col, one 8-byte store
+  barrier_lds_no_dma();              // the helpers' K^T and P' tiles are in LDS
+
+  // S <- e^gamma_C S + K^T (ks (.) Delta), key tile t, and
+  // O^T = rq (.) (qs (.) S^T Q^T + Delta^T P'^T): lane (m, g) ends with
+  // columns 32 w + 16 h + 8 g .. + 7 of token 32 R + m, a 16-byte store each.
+  // Eight groups of products, each two key tiles' of one token block and one
+  // of O's six lower blocks (three independent chains), their operands read a
+  // group ahead.
+  const float gl = Sc->row[kRowGl];
+  float qs[2], rq[2];
   if constexpr (OUT) {
-    uint16_t* const obase = cx.out + (static_cast<size_t>(t0) * cx.HV + cx.hv) * kDim;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if (r < 2) read_p(r + 2);
-      o[r] = o[r] * (cx.scale * B->slot[kSlotEg + r * 16 + col]);
+    for (int R = 0; R < 2; ++R) {
+      qs[R] = Sc->row[kRowEg + 32 * R + m];
+      if constexpr (L2) rq[R] = Qn[32 * R + m];
+    }
+  }
+  // O's blocks in the order of the groups: (R, kb)
+  constexpr int kOR[6] = {0, 1, 0, 1, 1, 1}, kOKb[6] = {0, 0, 1, 1, 2, 3};
+  s16x8 ktop[2][2], pop[2][2];
+  auto read_group = [&](int i, int set) {
 #pragma unroll
-      for (int kb = 0; kb <= (r >> 1); ++kb) {
-        const int b = tri_blk(r, kb);
-        o[r] = mfma_bf16(dh[kb], ph[b], o[r]);
-        o[r] = mfma_bf16(dh[kb], pl[b], o[r]);
-        o[r] = mfma_bf16(dl[kb], ph[b], o[r]);
+    for (int u = 0; u < 2; ++u)
+      ktop[set][u] = ld_op(&Kt[((2 * (i >> 2) + u) * 4 + (i & 3)) * kBlk + lane * 8]);
+    if constexpr (OUT) {
+      if (i < 6) {
+        const int blk = tri_blk(kOR[i], kOKb[i]);
+        pop[set][0] = ld_op(&Pb[blk * kBlk + lane * 8]);
+        pop[set][1] = ld_op(&Pb[(kTriBlocks + blk) * kBlk + lane * 8]);
       }
-      if constexpr (L2) o[r] = o[r] * Qn[r * 16 + col];
-      const int tok = r * 16 + col;
-      const u32x2 ob = {pack_bf16x2(o[r][0], o[r][1]), pack_bf16x2(o[r][2], o[r][3])};
-      if (tok < n)
-        *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(obase) +
-                                  row_bytes(tok, cx.vstep, cw * 16 + g4 * 4)) = ob;
     }
+  };
+  auto store_o = [&](int R) {
+    const int c0 = cx.start + ci * kChunk;
+    const int tok = 32 * R + m;
+    if constexpr (L2) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[R][r] *= rq[R];
+    }
+    if (!LAST || tok < cx.end - c0) {
+      char* const dst = reinterpret_cast<char*>(
+                            cx.out + (static_cast<size_t>(c0) * cx.HV + cx.hv) * kDim) +
+                        row_bytes(tok, cx.vstep, 32 * wave + 8 * g);
+      *reinterpret_cast<s16x8*>(dst) = to_bf16x8<0>(o[R]);
+      *reinterpret_cast<s16x8*>(dst + 32) = to_bf16x8<1>(o[R]);
+    }
+  };
+  read_group(0, 0);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int set = i & 1, t = 2 * (i >> 2), kb = i & 3;
+    if (i < 7) read_group(i + 1, set ^ 1);
+    if (kb == 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st[t + u][r] *= gl;
+    }
+    if constexpr (OUT) {
+      if (i < 2) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] *= qs[i];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) st[t + u] = mfma32_bf16(ktop[set][u], eh[kb], st[t + u]);
+    if constexpr (OUT) {
+      if (i < 6) o[kOR[i]] = mfma32_bf16(dh[kOKb[i]], pop[set][0], o[kOR[i]]);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) st[t + u] = mfma32_bf16(ktop[set][u], el[kb], st[t + u]);
+    if constexpr (OUT) {
+      if (i < 6) {
+        o[kOR[i]] = mfma32_bf16(dh[kOKb[i]], pop[set][1], o[kOR[i]]);
+        o[kOR[i]] = mfma32_bf16(dl[kOKb[i]], pop[set][0], o[kOR[i]]);
+      }
+      if (i == 4) store_o(0);
+      if (i == 6) store_o(1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
 
-  // S <- e^gamma_C S + K^T (ks (.) Delta), key tile t
-  const float gl = B->slot[kSlotGl];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    if (t == 1) read_kt(4);
-    f32x4 acc = st[t] * gl;
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      acc = mfma_bf16(kt_op[t][kb], eh[kb], acc);
-      acc = mfma_bf16(kt_op[t][kb], el[kb], acc);
-    }
-    st[t] = acc;
-  }
-
-  wait_vmem();                       // the next chunk's DMA has landed
-  block_sync_lds();                  // for every wave; this chunk's LDS reads are done
-}
+  if constexpr (!LAST) barrier_lds_no_dma();   // the next chunk's inputs have landed; this
+}                                              // one's LDS reads are done
 
 // The end state of a scan: k-last fp32 (element (k, c) at c * 128 + k), or,
 // for a transition M (identity start), as the A operand blocks of the
-// combine's product M S: for row tile t and column block kb, 64 lanes x 8
-// bf16, hi then lo (block ((t * 4 + kb) * 2 + hl) * 512).  Column wave w
-// (cw: the wave's columns 16 w .. 16 w + 15) is half w % 2 of block kb = w /
-// 2: the selector products of its state read as an operand with the columns
-// as rows give lane (col, g) the columns 16 w + 4 g + e of row state_key(t,
-// col / 4) + col % 4, items 4 (w % 2) .. + 3 of the block's lane; those
-// columns started from start keys 32 kb + 8 g + item, the key order of the
-// combine's S operand.
-__device__ __forceinline__ void store_end(float* st_out, bool transition, const f32x4 (&st)[8],
-                                          const s16x8 (&sels)[2], int cw) {
-  const int lane = threadIdx.x & 63;
-  const int wave = cw;
-  const int col = lane & 15;
-  const int g4 = lane >> 4;
+// combine's product M S (16x16x32): for row tile t and column block kb, 64
+// lanes x 8 bf16, hi then lo (block ((t * 4 + kb) * 2 + hl) * 512).  Wave w's
+// columns are block kb = w: the selector products of its state read as an
+// operand with the columns as rows give lane (m, g) the columns 32 w + 16 h +
+// 8 g .. + 7 of key 32 t2 + perm32(m), the 8 items (lane group 2 h + g) of the
+// combine's row i of tile t, 32 (t / 2) + 8 (i / 4) + 4 (t % 2) + i % 4 being
+// that key (state_key).
+__device__ __forceinline__ void store_end(float* st_out, bool transition, const f32x16 (&st)[4],
+                                          const s16x8 (&sel)[2]) {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));      // as in scan_chunk
+  const int wave = wave_index();
+  const int m = lane & 31;
+  const int g = lane >> 5;
   if (!transition) {
+    float* const dst = st_out + static_cast<size_t>(32 * wave + perm32(m)) * kDim + 8 * g;
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
-      *reinterpret_cast<f32x4*>(st_out + static_cast<size_t>(wave * 16 + col) * kDim +
-                                state_key(t, g4)) = st[t];
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(dst + 32 * t + 16 * (q >> 1) + 4 * (q & 1)) =
+            f32x4{st[t][4 * q], st[t][4 * q + 1], st[t][4 * q + 2], st[t][4 * q + 3]};
     return;
   }
   uint16_t* ma = reinterpret_cast<uint16_t*>(st_out);
+  const int key = perm32(m);
+  const int tb = (key >> 2) & 1, i = 4 * (key >> 3) + (key & 3);
 #pragma unroll
-  for (int kb2 = 0; kb2 < 4; ++kb2) {                 // rows 32 kb2 .. 32 kb2 + 31
-    s16x8 al;
-    const s16x8 ah = split_hi_lo(st[2 * kb2], st[2 * kb2 + 1], al);
+  for (int t2 = 0; t2 < 4; ++t2) {
+    s16x8 hi[2], lo[2];
+    hi[0] = split8<0>(st[t2], lo[0]);
+    hi[1] = split8<1>(st[t2], lo[1]);
+    f32x16 mh, ml;
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const int t = 2 * kb2 + hf;
-      const int blk0 = (t * 4 + (wave >> 1)) * 2;
-      const int item = lane * 8 + (wave & 1) * 4;
-      *reinterpret_cast<s16x4*>(ma + blk0 * kBlk + item) =
-          to_bf16x4(mfma_bf16(ah, sels[hf], f32x4{0, 0, 0, 0}));
-      *reinterpret_cast<s16x4*>(ma + (blk0 + 1) * kBlk + item) =
-          to_bf16x4(mfma_bf16(al, sels[hf], f32x4{0, 0, 0, 0}));
+    for (int r = 0; r < 16; ++r) mh[r] = ml[r] = 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      mh = mfma32_bf16(hi[h], sel[h], mh);
+      ml = mfma32_bf16(lo[h], sel[h], ml);
     }
+    uint16_t* const blk = ma + ((2 * t2 + tb) * 4 + wave) * 2 * kBlk;
+    uint16_t* const d0 = blk + (i + 16 * g) * 8;
+    uint16_t* const d1 = blk + (i + 16 * (2 + g)) * 8;
+    *reinterpret_cast<s16x8*>(d0) = to_bf16x8<0>(mh);
+    *reinterpret_cast<s16x8*>(d1) = to_bf16x8<1>(mh);
+    *reinterpret_cast<s16x8*>(d0 + kBlk) = to_bf16x8<0>(ml);
+    *reinterpret_cast<s16x8*>(d1 + kBlk) = to_bf16x8<1>(ml);
   }
 }
 
-// Grid: (unit, q/k head) pairs in groups of 8 times the GVA ratio times the
-// column halves (W = 4: 2, W = 8: 1).  Workgroup b serves pair 8 (b / (8
-// ratio halves)) + b % 8 and, with m = (b / 8) % (ratio halves), its v-head
-// m % ratio and half m / ratio: the workgroups that read the same K and Q
-// are dispatched 8 apart, all to XCD b % 8 (workgroups go to the XCDs
-// round-robin), and share its L2 copy.  A unit is a sequence, or with SEG a role of one segment of
-// sequence 0.  The first segment launch (OUT false, no outputs) runs
+// Grid: (unit, q/k head) pairs in groups of 8 times the GVA ratio.  Workgroup
+// b serves pair 8 (b / (8 ratio)) + b % 8 and v-head (b / 8) % ratio of its
+// q/k head: the workgroups that read the same K and Q are dispatched 8 apart,
+// all to XCD b % 8 (workgroups go to the XCDs round-robin), and share its L2
+// copy.  A unit is a sequence, or with SEG a role of one segment of a
+// sequence.  The first segment launch (OUT false, no outputs) runs
 // segment 0 from the sequence's state (end: seg_S[1]) and segments
 // 1 .. nseg-2 from a zero start (end: seg_B) and from the identity without
 // values (end: seg_M, as the combine's operand); the second (OUT) runs every
 // segment from its start (segment 0: the sequence's state, then seg_S) with
 // the outputs, the last one's end being the new state.
-template <bool FEW, bool SEG, bool OUT, bool L2, int W, bool FUSE>
+template <bool FEW, bool SEG, bool OUT, bool L2, bool FUSE>
 __device__ __forceinline__ void scan_body(Params p) {
   static_assert(OUT || SEG, "only segments run without outputs");
-  static_assert(!FUSE || (!FEW && !SEG && OUT && W == kThreads / 64),
-                "the one-chunk kernel: half-state workgroups of the preparation's width");
+  static_assert(!FUSE || (!FEW && !SEG && OUT), "the one-chunk kernel runs plain scans");
   static_assert(OUT || !L2, "the L2-norm scales outputs only");
-  static_assert(W == kScanWaves || (W == kScanWaves / 2 && !SEG),
-                "half-state workgroups run plain scans only");
-  constexpr int kHalves = kScanWaves / W;
   // separate LDS objects, so that the compiler sees that the DMA into one
-  // buffer never writes what the chunk reads from the other
-  __shared__ ScanBuf<OUT> L0, L1;
+  // never writes what the chunk reads from another
+  __shared__ ScanIn<OUT> In0, In1;
+  __shared__ ScanScales S0, S1;
   __shared__ __attribute__((aligned(16))) uint16_t Kt[kKtElems];
   __shared__ __attribute__((aligned(16))) uint16_t Pb[OUT ? kPElems : 8];
   __shared__ float Qn[L2 ? kChunk : 1];    // 1 / |q_i| of the chunk's Q rows (L2-norm)
+  __shared__ __attribute__((aligned(16))) uint16_t Sel[2 * kBlk];   // the selectors
   const long long b = blockIdx.x;
   const int ratio = p.ratio;
-  const long long pair = (b / (8LL * ratio * kHalves)) * 8 + (b & 7);
-  const int member = static_cast<int>((b >> 3) % (ratio * kHalves));
-  const int jr = member % ratio;
-  const int cw0 = W == kScanWaves ? 0 : (member / ratio) * W;   // the first wave's column wave
+  const long long pair = (b / (8LL * ratio)) * 8 + (b & 7);
+  const int jr = static_cast<int>((b >> 3) % ratio);
   // units the grid covers: with SEG the launch's bound, each workgroup
   // finding its sequence's segment below (those past the batch's exit)
   const long long units = SEG ? (OUT ? p.nseg : seg_units1(p.nseg, p.N))
@@ -1520,8 +1549,8 @@ __device__ __forceinline__ void scan_body(Params p) {
   const int hv = h * ratio + jr;
   const int lane = threadIdx.x & 63;
   const int wave = wave_index();
-  const int col = lane & 15;
-  const int g4 = lane >> 4;
+  const int m = lane & 31;
+  const int g = lane >> 5;
   const size_t blk = static_cast<size_t>(kDim) * kDim;
 
   // role: start state, values, where the end state goes
@@ -1556,7 +1585,9 @@ __device__ __forceinline__ void scan_body(Params p) {
     start = __builtin_amdgcn_readlane(f.start, s);
     end = __builtin_amdgcn_readlane(f.end, s);
     const size_t sh = static_cast<size_t>(s) * p.HV + hv;        // the sequence's state
-    auto seg_blk = [&](float* base, int g) { return base + (static_cast<size_t>(g) * p.HV + hv) * blk; };
+    auto seg_blk = [&](float* base, int sg) {
+      return base + (static_cast<size_t>(sg) * p.HV + hv) * blk;
+    };
     int j;
     if (!OUT) {
       const int mid = nseg - 2;                   // segments 1 .. nseg-2
@@ -1599,48 +1630,54 @@ __device__ __forceinline__ void scan_body(Params p) {
       seq_slots(s, slot0, nchunks);
   }
 
-  // state registers (keys in the order of state_key); k-last storage: 4
-  // consecutive keys are one 16-byte vector.  The identity start of a
-  // transition gives column 16 w + m the unit vector of the key in register
-  // position (w, m): key state_key(w, m / 4) + m % 4, so that its end column
-  // is that start key's column of M, in the key order of the combine's
-  // operand.  (w: the column wave, cw0 + wave.)
-  f32x4 st[8];
-  const int cw = cw0 + wave;
-  const int c = cw * 16 + col;
+  // state registers; k-last storage: 8 consecutive keys are two 16-byte
+  // vectors.  The identity start of a transition gives column c the unit
+  // vector of key c, so that its end column is that start key's column of M.
+  f32x16 st[4];
+  const int c = 32 * wave + perm32(m);
+  const bool load_state = st_in != nullptr && (end > start || pass_through) &&
+                          (FUSE || wave < kScanWaves);   // helper waves hold no columns
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    st[t] = st_in != nullptr && (end > start || pass_through)
-                ? *reinterpret_cast<const f32x4*>(st_in + static_cast<size_t>(c) * kDim +
-                                                  state_key(t, g4))
-                : f32x4{0, 0, 0, 0};
-    if (identity) {
+  for (int t = 0; t < 4; ++t) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) st[t][e] = t == cw && 4 * g4 + e == col ? 1.0f : 0.0f;
+    for (int q = 0; q < 4; ++q) {
+      const int key = 32 * t + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
+      const f32x4 v = load_state ? *reinterpret_cast<const f32x4*>(
+                                       st_in + static_cast<size_t>(c) * kDim + key)
+                                 : f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        st[t][4 * q + e] = identity ? (key + e == c ? 1.0f : 0.0f) : v[e];
     }
   }
-  // selector operands: Sel_h[k][j] = (k == 16 h + j) over a 32-long k block
-  s16x8 sels[2];
+  // selector operands: Sel_h[k][j] = (16 h + k == perm32(j)) over a 16-long k
+  // block
+  s16x8 sel[2];
 #pragma unroll
-  for (int hf = 0; hf < 2; ++hf)
+  for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      sels[hf][e] = (e == 4 * hf + (col & 3) && g4 == (col >> 2)) ? 0x3f80 : 0;
+    for (int e = 0; e < 8; ++e) sel[h2][e] = perm32(m) == 16 * h2 + 8 * g + e ? 0x3f80 : 0;
 
   // No tokens: a sequence ends in zeros, as the reference; a segment with no
   // chunk slots (a malformed batch whose slots ran past the workspace's)
   // passes its start through (transition: the identity, zero-start end:
   // zeros), and so does the sequence's end state.
   if (nchunks <= 0) {
-    if (st_out != nullptr) {
+    if (st_out != nullptr && wave < kScanWaves) {
       if (!SEG) {
 #pragma unroll
-        for (int t = 0; t < 8; ++t) st[t] = f32x4{0, 0, 0, 0};
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) st[t][r] = 0.0f;
       }
-      store_end(st_out, identity, st, sels, cw);
+      store_end(st_out, identity, st, sel);
     }
     return;
   }
+  start = uniform(start);
+  end = uniform(end);
+  nchunks = uniform(nchunks);
+  slot0 = uniform(slot0);
   ScanCtx cx;
   cx.k = p.k;
   cx.q = p.q;
@@ -1658,49 +1695,61 @@ __device__ __forceinline__ void scan_body(Params p) {
   cx.h = h;
   cx.hv = hv;
   cx.values = values;
-  cx.scale = p.scale;
-  cx.cw0 = cw0;
 
-  const s16x8 sel = sels[wave & 1];       // this wave's half of a 32-key / 32-column block
-  u32x2 vnext[4];
+  const ChunkSrc first_src = chunk_src(cx, 0);
+  if (wave < 2) *reinterpret_cast<s16x8*>(&Sel[wave * kBlk + lane * 8]) = sel[wave];
   if constexpr (FUSE) {
-    // The chunk's K and Q rows by DMA and its V while this workgroup prepares
-    // its slot in LDS (the preparation's LDS in the second buffer, which one
-    // chunk never uses), then its one chunk step.
-    static_assert(sizeof(PrepLds) <= sizeof(ScanBuf<OUT>), "the preparation fits a buffer");
-    scan_issue<OUT, W, false>(&L0, cx, 0, vnext);
-    prep_chunk<true>(p, 0, start, end - start, hv, h, 1, *reinterpret_cast<PrepLds*>(&L1),
-                     L0.slot);
+    // The chunk's K and Q rows by DMA while this workgroup (four waves, each
+    // main and helper in turn) prepares its slot in LDS, then its one chunk
+    // step.
+    static_assert(sizeof(PrepLds) <= sizeof(ScanIn<OUT>), "the preparation fits a buffer");
+#pragma unroll
+    for (int part = 0; part < 4; ++part)
+      issue_part<OUT, false>(&In0, &S0, cx, first_src, part, wave, lane);
+    prep_chunk<true>(p, 0, start, end - start, hv, h, 1, *reinterpret_cast<PrepLds*>(&In1), In0.T,
+                     S0.row);
     wait_vmem();
     block_sync_lds();
-    scan_chunk<OUT, L2, W, true>(&L0, &L1, Kt, Pb, Qn, cx, st, vnext, sel, 0);
-    if (st_out != nullptr) store_end(st_out, identity, st, sels, cw);
+    side_tiles<OUT, L2>(&In0, &S0, Kt, Pb, Qn, Sel, wave, lane);
+    scan_chunk<OUT, L2, true>(&In0, &S0, Kt, Pb, Qn, cx, st, Sel, 0);
+    if (st_out != nullptr) store_end(st_out, identity, st, sel);
     return;
   }
-  scan_issue<OUT, W>(&L0, cx, 0, vnext);
-  wait_vmem();
-  block_sync_lds();
-  for (int ci = 0; ci < nchunks; ci += 2) {
-    scan_chunk<OUT, L2, W>(&L0, &L1, Kt, Pb, Qn, cx, st, vnext, sel, ci);
-    if (ci + 1 < nchunks)                                                      // uniform
-      scan_chunk<OUT, L2, W>(&L1, &L0, Kt, Pb, Qn, cx, st, vnext, sel, ci + 1);
+  if (wave >= kScanWaves) {                                                    // uniform
+#pragma unroll
+    for (int part = 0; part < 4; ++part)
+      issue_part<OUT>(&In0, &S0, cx, first_src, part, wave - kScanWaves, lane);
+    wait_vmem();
+    barrier_lds_no_dma();
+    for (int ci = 0; ci < nchunks; ci += 2) {
+      help_chunk<OUT, L2>(&In0, &S0, &In1, &S1, Kt, Pb, Qn, cx, Sel, ci);
+      if (ci + 1 < nchunks)                                                    // uniform
+        help_chunk<OUT, L2>(&In1, &S1, &In0, &S0, Kt, Pb, Qn, cx, Sel, ci + 1);
+    }
+    return;
   }
-  if (st_out != nullptr) store_end(st_out, identity, st, sels, cw);
+  wait_vmem();                       // the state, here rather than in each chunk step
+  barrier_lds_no_dma();
+  for (int ci = 0; ci < nchunks - 1; ++ci)
+    scan_chunk<OUT, L2, false>((ci & 1) ? &In1 : &In0, (ci & 1) ? &S1 : &S0, Kt, Pb, Qn, cx, st,
+                               Sel, ci);
+  scan_chunk<OUT, L2, true>((nchunks & 1) ? &In0 : &In1, (nchunks & 1) ? &S0 : &S1, Kt, Pb, Qn,
+                            cx, st, Sel, nchunks - 1);
+  if (st_out != nullptr) store_end(st_out, identity, st, sel);
 }
 
-template <bool FEW, bool SEG, bool OUT, bool L2, int W>
-__global__ __launch_bounds__(64 * W)
-__attribute__((amdgpu_waves_per_eu(W == kScanWaves ? 2 : 1, W == kScanWaves ? 2 : 1)))
+template <bool FEW, bool SEG, bool OUT, bool L2>
+__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void scan_kernel(Params p) {
-  scan_body<FEW, SEG, OUT, L2, W, false>(p);
+  scan_body<FEW, SEG, OUT, L2, false>(p);
 }
 
-// Prefills whose tokens all fit one chunk: each (sequence, v-head, half)
+// Prefills whose tokens all fit one chunk: each (sequence, v-head)
 // workgroup prepares its sequence's chunk in LDS and scans it, in one launch.
 template <bool L2>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void one_chunk_kernel(Params p) {
-  scan_body<false, false, true, L2, kThreads / 64, true>(p);
+  scan_body<false, false, true, L2, true>(p);
 }
 
 // ---------------------------------------------------------------------------
@@ -1711,7 +1760,7 @@ void one_chunk_kernel(Params p) {
 // hi/lo) and zero-start end B_j.  Combine: S_{j+1} = M_j S_j + B_j for j = 1
 // .. nseg-2, segment after segment, as bf16 MFMA with S_j split into hi + lo.
 // One workgroup per (sequence, v-head, 16 state columns); wave w computes row
-// tile w (in the scan's key order: rows state_key(w, i / 4) + i % 4, the rows
+// tile w (rows state_key(w, i / 4) + i % 4, the rows
 // of M's tile w) and hands its rows of S_j to the other waves as half of the
 // B operand's k block w / 2 through LDS (two buffers: one barrier a step).  A step is short (12 MFMAs a wave), so each wave's M
 // blocks and B tile are loaded three steps ahead, into three register sets
@@ -1862,18 +1911,13 @@ SegPlan seg_plan(long long L, long long N, long long HV) {
   return best;
 }
 
-// A plain scan whose whole-state workgroups (N HV) would fill at most half
-// the CUs runs as half-state workgroups of 4 waves (two per (sequence,
-// v-head), one wave a SIMD): chunk steps at about half the cost.
-bool half_state_scan(long long N, long long HV) { return N >= 1 && 2 * N * HV <= kCUs; }
-
 // Prefills past the token path whose tokens all fit one chunk (so every
-// sequence is one chunk), with half-state workgroups that fit the GPU at
-// once: one launch in which each (sequence, v-head, half) workgroup prepares
-// its chunk in LDS and scans it -- no workspace round trip and one launch
-// instead of the preparation's and the scan's.
+// sequence is one chunk) and whose workgroups fill at most half the CUs: one
+// launch in which each (sequence, v-head) workgroup prepares its chunk in LDS
+// and scans it -- no workspace round trip and one launch instead of the
+// preparation's and the scan's.
 bool fused_prefill(long long L, long long N, long long HV) {
-  return L > kSmallTokens && L <= kChunk && half_state_scan(N, HV);
+  return L > kSmallTokens && L <= kChunk && N >= 1 && 2 * N * HV <= kCUs;
 }
 
 bool use_segments(long long L, long long N, long long HV) {
@@ -2097,10 +2141,10 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
     if (e == hipSuccess) e = mark(3);
     return e;
   }
-  // One workgroup per (sequence or segment role, v-head, column half), in
-  // groups of 8 (unit, q/k head) pairs times the GVA ratio times the halves.
-  auto scan_grid = [&](long long units, int halves) {
-    return dim3(static_cast<unsigned>((units * H + 7) / 8 * 8 * p.ratio * halves));
+  // One workgroup per (sequence or segment role, v-head), in groups of 8
+  // (unit, q/k head) pairs times the GVA ratio.
+  auto scan_grid = [&](long long units) {
+    return dim3(static_cast<unsigned>((units * H + 7) / 8 * 8 * p.ratio));
   };
   if (fused_prefill(total_seq_len, num_seqs, HV)) {
     // one launch (the timed form's intervals as on the token path)
@@ -2109,10 +2153,8 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
     if (e == hipSuccess) e = mark(2);
     if (e != hipSuccess) return e;
     p.short_limit = 0;
-    constexpr int kHalfW = kScanWaves / 2;
-    static_assert(kHalfW == kThreads / 64, "the one-chunk kernel's workgroups are half-state");
     auto* fused = p.l2norm ? one_chunk_kernel<true> : one_chunk_kernel<false>;
-    hipLaunchKernelGGL(fused, scan_grid(num_seqs, 2), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL(fused, scan_grid(num_seqs), dim3(kThreads), 0, stream, p);
     e = hipGetLastError();
     if (e == hipSuccess) e = mark(3);
     return e;
@@ -2148,9 +2190,9 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
     // segments: transitions and zero-start ends, the starts, then every
     // segment with its outputs (grids: the workspace's segments bound the
     // batch's units; workgroups past them exit)
-    auto* scan1 = p.few ? scan_kernel<true, true, false, false, kScanWaves>
-                        : scan_kernel<false, true, false, false, kScanWaves>;
-    hipLaunchKernelGGL(scan1, scan_grid(seg_units1(p.nseg, num_seqs), 1), dim3(kScanThreads), 0,
+    auto* scan1 = p.few ? scan_kernel<true, true, false, false>
+                        : scan_kernel<false, true, false, false>;
+    hipLaunchKernelGGL(scan1, scan_grid(seg_units1(p.nseg, num_seqs)), dim3(kScanThreads), 0,
                        stream, p);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -2159,24 +2201,17 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
                        dim3(64 * kCombWaves), 0, stream, p);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    auto* scan = p.few ? (p.l2norm ? scan_kernel<true, true, true, true, kScanWaves>
-                                   : scan_kernel<true, true, true, false, kScanWaves>)
-                       : (p.l2norm ? scan_kernel<false, true, true, true, kScanWaves>
-                                   : scan_kernel<false, true, true, false, kScanWaves>);
-    hipLaunchKernelGGL(scan, scan_grid(p.nseg, 1), dim3(kScanThreads), 0, stream, p);
-  } else if (half_state_scan(num_seqs, HV)) {
-    constexpr int kHalfW = kScanWaves / 2;
-    auto* scan = p.few ? (p.l2norm ? scan_kernel<true, false, true, true, kHalfW>
-                                   : scan_kernel<true, false, true, false, kHalfW>)
-                       : (p.l2norm ? scan_kernel<false, false, true, true, kHalfW>
-                                   : scan_kernel<false, false, true, false, kHalfW>);
-    hipLaunchKernelGGL(scan, scan_grid(num_seqs, 2), dim3(64 * kHalfW), 0, stream, p);
+    auto* scan = p.few ? (p.l2norm ? scan_kernel<true, true, true, true>
+                                   : scan_kernel<true, true, true, false>)
+                       : (p.l2norm ? scan_kernel<false, true, true, true>
+                                   : scan_kernel<false, true, true, false>);
+    hipLaunchKernelGGL(scan, scan_grid(p.nseg), dim3(kScanThreads), 0, stream, p);
   } else {
-    auto* scan = p.few ? (p.l2norm ? scan_kernel<true, false, true, true, kScanWaves>
-                                   : scan_kernel<true, false, true, false, kScanWaves>)
-                       : (p.l2norm ? scan_kernel<false, false, true, true, kScanWaves>
-                                   : scan_kernel<false, false, true, false, kScanWaves>);
-    hipLaunchKernelGGL(scan, scan_grid(num_seqs, 1), dim3(kScanThreads), 0, stream, p);
+    auto* scan = p.few ? (p.l2norm ? scan_kernel<true, false, true, true>
+                                   : scan_kernel<true, false, true, false>)
+                       : (p.l2norm ? scan_kernel<false, false, true, true>
+                                   : scan_kernel<false, false, true, false>);
+    hipLaunchKernelGGL(scan, scan_grid(num_seqs), dim3(kScanThreads), 0, stream, p);
   }
   e = hipGetLastError();
   if (e == hipSuccess) e = mark(3);
