@@ -425,6 +425,119 @@ hipError_t launch(const StepArgs& s, hipStream_t stream, hipEvent_t start_event,
   return hipSuccess;
 }
 
+// Layers in one launch: plans that gdn_decode_graph_create records run as
+// one grid when nothing orders them -- the same sizes, state type, flag and
+// scale (one kernel, one grid), one token and a state to read (the
+// single-token kernel), and no buffer one of them writes read or written by
+// another.
+struct Range {
+  uintptr_t lo, hi;
+};
+inline bool overlaps(const Range& x, const Range& y) { return x.lo < y.hi && y.lo < x.hi; }
+
+// The byte ranges a step reads (first eight) and writes (last two).
+void step_ranges(const StepArgs& s, Range (&r)[10]) {
+  const size_t B = s.B, T = s.T, H = s.H, HV = s.HV;
+  const size_t state = B * HV * kDim * kDim * (s.state_bf16 ? 2 : 4);
+  const size_t qk = B * T * H * kDim * 2, vo = B * T * HV * kDim * 2, gate = B * T * HV * 2;
+  const void* p[10] = {s.q, s.k, s.v, s.state, s.A_log, s.a, s.dt_bias, s.b, s.output, s.new_state};
+  const size_t n[10] = {qk, qk, vo, state, HV * 4, gate, HV * 4, gate, vo, state};
+  for (int i = 0; i < 10; ++i) {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(p[i]);
+    r[i] = Range{lo, p[i] == nullptr ? lo : lo + n[i]};
+  }
+}
+
+bool groupable(const StepArgs& s) {
+  return s.T == 1 && s.state != nullptr && s.B > 0;
+}
+
+bool same_grid(const StepArgs& x, const StepArgs& y) {
+  return x.B == y.B && x.H == y.H && x.HV == y.HV && x.state_bf16 == y.state_bf16 &&
+         (x.use_qk_l2norm != 0) == (y.use_qk_l2norm != 0) && x.scale == y.scale;
+}
+
+bool independent(const StepArgs& x, const StepArgs& y) {
+  Range rx[10], ry[10];
+  step_ranges(x, rx);
+  step_ranges(y, ry);
+  for (int w = 8; w < 10; ++w)
+    for (int i = 0; i < 10; ++i)
+      if (overlaps(rx[w], ry[i]) || overlaps(ry[w], rx[i])) return false;
+  return true;
+}
+
+// Layers of args[0 .. n-1] that one launch takes, from the first on; 1: the
+// first alone, by its own kernel.
+int group_layers(const StepArgs* const* args, int n) {
+  const StepArgs& s = *args[0];
+  if (!groupable(s)) return 1;
+  int count = 1;
+  while (count < n && count < kMaxLayers) {
+    const StepArgs& next = *args[count];
+    if (!groupable(next) || !same_grid(s, next)) break;
+    bool free = true;
+    for (int i = 0; i < count && free; ++i) free = independent(*args[i], next);
+    if (!free) break;
+    ++count;
+  }
+  // one launch's grid: z at most 65535 sequences, work-items in 32 bits
+  // (with the widest workgroups of a head, 64 threads a row group)
+  const long long per_layer = static_cast<long long>(s.B) * s.HV * kDim / kLaneGroups * 64;
+  while (count > 1 && (static_cast<long long>(count) * s.B > 65535 ||
+                       count * per_layer > (1LL << 31) - 1))
+    --count;
+  return count;
+}
+
+template <int NS, int W, bool BF16>
+hipError_t launch_layers_one(const StepArgs& s, int count, const LayerTable& t, hipStream_t stream) {
+  const unsigned ratio = static_cast<unsigned>(s.HV / s.H);
+  const unsigned z = static_cast<unsigned>(count) * static_cast<unsigned>(s.B);
+  const dim3 grid(ratio * (kDim / (kLaneGroups * NS * W)), static_cast<unsigned>(s.H), z);
+  auto* kern = s.use_qk_l2norm != 0 ? gdn_decode_layers_k128<NS, W, true, BF16>
+                                    : gdn_decode_layers_k128<NS, W, false, BF16>;
+  const unsigned h_ratio = static_cast<unsigned>(s.H) | (ratio << 16) |
+                           (z >= kGroupMinSeqs ? kGroupFlag : 0u);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * W), 0, stream, h_ratio, s.B, s.scale, t);
+  return hipGetLastError();
+}
+
+// The layers' launch, with the single-token launch shape of all their heads
+// together.
+hipError_t launch_layers(const StepArgs* const* args, int count, hipStream_t stream) {
+  const StepArgs& s = *args[0];
+  LayerTable t{};
+  for (int i = 0; i < count; ++i) {
+    const StepArgs& l = *args[i];
+    t.layer[i] = LayerArgs{l.state, static_cast<const uint16_t*>(l.q),
+                           static_cast<const uint16_t*>(l.k), static_cast<const uint16_t*>(l.v),
+                           static_cast<const uint16_t*>(l.a), static_cast<const uint16_t*>(l.b),
+                           l.A_log, l.dt_bias, static_cast<uint16_t*>(l.output), l.new_state};
+  }
+  int ns = 0, w = 0, policy = 0;
+  choose_shape(static_cast<long long>(count) * s.B * s.HV, s.state_bf16 != 0, 1, &ns, &w, &policy);
+  if (s.state_bf16 == 0) {
+    switch (ns * 16 + w) {                         // the rows of kShapeFp32
+      case 1 * 16 + 1: return launch_layers_one<1, 1, false>(s, count, t, stream);
+      case 2 * 16 + 2: return launch_layers_one<2, 2, false>(s, count, t, stream);
+      case 4 * 16 + 1: return launch_layers_one<4, 1, false>(s, count, t, stream);
+      case 8 * 16 + 1: return launch_layers_one<8, 1, false>(s, count, t, stream);
+      case 2 * 16 + 4: return launch_layers_one<2, 4, false>(s, count, t, stream);
+      default: return hipErrorInvalidValue;
+    }
+  }
+  switch (ns * 16 + w) {                           // the rows of kShapeBf16
+    case 1 * 16 + 2: return launch_layers_one<1, 2, true>(s, count, t, stream);
+    case 1 * 16 + 4: return launch_layers_one<1, 4, true>(s, count, t, stream);
+    case 2 * 16 + 4: return launch_layers_one<2, 4, true>(s, count, t, stream);
+    case 2 * 16 + 2: return launch_layers_one<2, 2, true>(s, count, t, stream);
+    case 2 * 16 + 1: return launch_layers_one<2, 1, true>(s, count, t, stream);
+    case 4 * 16 + 4: return launch_layers_one<4, 4, true>(s, count, t, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 StepArgs make_args(const void* q, const void* k, const void* v, const void* state,
                    const float* A_log, const void* a, const float* dt_bias, const void* b,
                    float scale, void* output, void* new_state, int B, int T, int H, int HV,
@@ -628,8 +741,18 @@ int gdn_decode_graph_create(const gdn_decode_plan* const* plans, int n,
   e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
   hipError_t launch_error = hipSuccess;
   if (e == hipSuccess) {
-    for (int i = 0; i < n && launch_error == hipSuccess; ++i)
-      launch_error = launch(plans[i]->args, s, nullptr, nullptr);
+    for (int i = 0; i < n && launch_error == hipSuccess;) {
+      const StepArgs* args[kMaxLayers];
+      int most = 0;
+      while (most < kMaxLayers && i + most < n && plans[i + most]->device == plans[i]->device) {
+        args[most] = &plans[i + most]->args;
+        ++most;
+      }
+      const int count = group_layers(args, most);
+      launch_error = count > 1 ? launch_layers(args, count, s)
+                               : launch(plans[i]->args, s, nullptr, nullptr);
+      i += count;
+    }
     hipGraph_t g = nullptr;
     e = hipStreamEndCapture(s, &g);   // always ends the capture, also after a failed launch
     if (e == hipSuccess && launch_error != hipSuccess) e = launch_error;

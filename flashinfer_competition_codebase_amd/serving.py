@@ -17,6 +17,10 @@ Here:
   layer) and runs them eagerly in one native call, or records them once in
   a HIP graph (``gdn_decode_graph_create``: stream capture on a private
   stream, no memset nodes) and replays it, one submission per model step.
+  In the graph, consecutive layers of the same sizes and scale whose buffers
+  no other one of them writes run as one launch (48 layers at B = 1, 16/32
+  heads: 37 us a replay, 122 us as one launch each); layers that share a
+  buffer keep their order.
 
 Both launch on torch's current stream of the plans' device; there is no
 CPU path.
@@ -134,8 +138,9 @@ class DecodeLayers:
             _lib.check(code, "gdn_decode_plan_run")
 
     def capture(self) -> None:
-        """Record every layer's step, in order, in one HIP graph (replaces a
-        previous one)."""
+        """Record every layer's step, in order (layers that share no written
+        buffer may run together), in one HIP graph (replaces a previous
+        one)."""
         self._check_open()
         self.release_graph()
         graph = ctypes.c_void_p()

@@ -183,7 +183,10 @@ int gdn_decode_plan_run(const gdn_decode_plan* const* plans, int n, void* hip_st
 void gdn_decode_plan_destroy(gdn_decode_plan* plan);
 
 /*
- * One HIP graph of the launches of plans[0 .. n-1] (n >= 1), in order,
+ * One HIP graph of the steps of plans[0 .. n-1] (n >= 1), in order -- up to
+ * 48 consecutive ones of the same sizes, state type, flag and scale, one
+ * token each, of which none writes what another reads or writes, as one
+ * launch --
  * recorded by stream capture on a private stream of the current device and
  * instantiated once; gdn_decode_graph_launch replays it on hip_stream (a
  * stream of the same device), as one submission for all n steps (e.g. the

@@ -204,3 +204,97 @@ def test_repeat_calls_reuse_the_validated_launch(hip_device):
     del out
     gc.collect()
     assert len(kmod._VALIDATED) == before - 1
+
+
+def _same_bits_graph_and_eager(make, n_steps=3, l2=True):
+    """The layers ``make()`` builds (fresh buffers, the same values each time)
+    replayed from a graph and run eagerly: every output and state the same
+    bits after each of ``n_steps`` steps, with new inputs between them."""
+    runs = []
+    for mode in ("eager", "graph"):
+        dev = make()
+        layers = DecodeLayers(dev, use_qk_l2norm=l2)
+        if mode == "graph":
+            layers.capture()
+        got = []
+        for step in range(n_steps):
+            if step > 0:
+                for d in dev:
+                    for n in INPUTS:
+                        d[n].copy_(d[n].roll(step, dims=0).neg())
+            layers.replay() if mode == "graph" else layers.run()
+            torch.cuda.synchronize()
+            got += [x.clone() for d in dev for x in (d["output"], d["new_state"])]
+        layers.close()
+        runs.append(got)
+    for i, (x, y) in enumerate(zip(*runs)):
+        assert torch.equal(x, y), f"buffer {i}"
+
+
+@pytest.mark.parametrize("n_layers,B,H,HV,dtype,l2", [
+    (50, 1, 16, 32, torch.float32, True),      # more layers than one launch takes (48)
+    (49, 1, 4, 8, torch.float32, False),       # ... with one left over
+    (2, 1, 1, 1, torch.float32, False),        # the fewest layers and heads
+    (5, 3, 3, 12, torch.float32, True),        # odd sequences, heads and GVA ratio
+    (9, 15, 2, 4, torch.float32, False),       # 135 sequences: grouped by XCD
+    (2, 1, 4, 8, torch.bfloat16, True),
+    (7, 2, 16, 32, torch.bfloat16, True),
+    (3, 40, 16, 32, torch.bfloat16, False),
+])
+def test_graph_of_equal_layers_matches_eager_bits(n_layers, B, H, HV, dtype, l2, hip_device):
+    """Layers of one size, each its own buffers, run as one launch in a graph
+    and one each eagerly: a row's arithmetic is the same in both."""
+    _announce(f"DecodeLayers equal layers: {n_layers} x B={B} qk{H}_v{HV} {dtype} l2={l2}")
+
+    def make():
+        dev = []
+        for i in range(n_layers):
+            t = make_inputs(B, H, HV, seed=5400 + i)
+            d = {n: (x.to(hip_device) if isinstance(x, torch.Tensor) else x)
+                 for n, x in t.items()}
+            d["state"] = d["state"].to(dtype)
+            d["new_state"] = d["state"] if i % 2 == 0 else torch.empty_like(d["state"])
+            d["output"] = torch.empty(B, 1, HV, 128, dtype=torch.bfloat16, device=hip_device)
+            dev.append(d)
+        return dev
+
+    _same_bits_graph_and_eager(make, l2=l2)
+
+
+@pytest.mark.parametrize("link", ["output_to_v", "shared_state", "shared_output", "scale",
+                                  "state_of_previous", "gates_in_state"])
+def test_graph_keeps_the_order_of_linked_layers(link, hip_device):
+    """Layers of one size where one reads or rewrites what another writes run
+    in their order in a graph, as eagerly (and layers with different scales
+    each use their own)."""
+    _announce(f"DecodeLayers linked layers: {link}")
+    B, H, HV, n_layers = 2, 4, 8, 6
+
+    def make():
+        dev = []
+        for i in range(n_layers):
+            t = make_inputs(B, H, HV, seed=5500 + i)
+            d = {n: (x.to(hip_device) if isinstance(x, torch.Tensor) else x)
+                 for n, x in t.items()}
+            d["new_state"] = d["state"]
+            d["output"] = torch.zeros(B, 1, HV, 128, dtype=torch.bfloat16, device=hip_device)
+            dev.append(d)
+        for i in range(1, n_layers):
+            prev, d = dev[i - 1], dev[i]
+            if link == "output_to_v":
+                d["v"] = prev["output"]
+            elif link == "shared_state" and i in (2, 3):
+                d["state"] = d["new_state"] = dev[0]["state"]
+            elif link == "shared_output" and i == 4:
+                d["output"] = dev[1]["output"]
+            elif link == "scale":
+                d["scale"] = 0.05 + 0.01 * (i // 2)
+            elif link == "state_of_previous":
+                d["state"] = prev["new_state"]
+                d["new_state"] = torch.zeros_like(d["state"])
+            elif link == "gates_in_state" and i == 3:
+                # dt_bias lives in a row of another layer's state
+                d["dt_bias"] = dev[2]["state"].view(-1)[:HV]
+        return dev
+
+    _same_bits_graph_and_eager(make, l2=False)
