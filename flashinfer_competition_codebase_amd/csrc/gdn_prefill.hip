@@ -39,15 +39,13 @@
 //      and writes each slot's sequence, first token and token count.  With
 //      one sequence, or a few (their slots found in the kernels), it is not
 //      launched.
-//   2. prep, grid (chunk slots, H) -- or (chunk slots, HV), one v-head a
-//      workgroup, when all of those fit on the GPU at once -- four
-//      workgroups per CU: what does not depend on the state, for all chunks
-//      at once -- K K^T (bf16 MFMA: the inputs are bf16, once per q/k head
-//      and workgroup), then per v-head the gates and
-//      gamma and T by block recursion (fp32 MFMA) -- into a 14 KiB workspace
-//      slot per (chunk, v-head): the lower blocks of T diag(beta), split
-//      into bf16 hi + lo in the order the scan's MFMAs read them, and the
-//      row scales.
+//   2. prep, one wave per (chunk slot, q/k head) -- or (chunk slot, v-head)
+//      when all of those fit on the GPU at once: what does not depend on the
+//      state, for all chunks at once -- K K^T (bf16 MFMA: the inputs are bf16,
+//      once per wave), then per v-head the gates and gamma and T by block
+//      recursion (fp32 MFMA) -- into a 14 KiB workspace slot per (chunk,
+//      v-head): the lower blocks of T diag(beta), split into bf16 hi + lo in
+//      the order the scan's MFMAs read them, and the row scales.
 //   3. scan, one workgroup per (sequence, v-head), XCD-aware order: the
 //      sequential part chunk after chunk.  Four main waves, one a SIMD, hold
 //      the whole 128 x 128 state in registers (32 columns each); four helper
@@ -144,20 +142,17 @@ bool maybe_all_short(long long L, long long N) {
   return L > kSmallTokens && N >= 2 && N <= kFewSeqs && L <= N * kSmallTokens;
 }
 constexpr float kL2Eps = 1e-6f;
-// v-heads of a GVA group whose gate inputs the preparation kernel loads with
-// the chunk's K rows (the others' when it reaches them).
-constexpr int kPrepGateHeads = 2;
-// A preparation workgroup takes a whole GVA group of v-heads (K K^T made
-// once for all of them, the v-heads one after another) unless one workgroup
-// per (slot, v-head) all fit on the GPU at once (4 a CU, 256 CUs): then each
-// takes one v-head, and the chain of one workgroup -- the preparation's time
-// on a grid that small -- is one v-head's (15k against 25k cycles at ratio 2).
-constexpr long long kPrepSplitMaxWorkgroups = 1024;
-inline bool prep_split(long long slots, int HV) {
-  return slots * HV <= kPrepSplitMaxWorkgroups;
-}
+// A preparation wave takes a whole GVA group of v-heads (K K^T made once for
+// all of them, the v-heads one after another) unless one wave per (slot,
+// v-head) all fit on the GPU at once (16 a CU, 256 CUs): then each takes one
+// v-head, and the chain of one wave -- the preparation's time on a grid that
+// small -- is one v-head's.
+constexpr long long kPrepSplitMaxWaves = 4096;
+constexpr long long kPrepSpreadMaxWaves = 1024;     // 4 a CU
+inline bool prep_split(long long slots, int HV) { return slots * HV <= kPrepSplitMaxWaves; }
 constexpr float kSoftplusThreshold = 20.0f;
 constexpr float kLog2e = 1.44269504088896341f;
+constexpr float kLn2 = 0.693147180559945309f;
 
 // Workspace slot of one (chunk, v-head), offsets in floats.  The scan's MFMA
 // operand T diag(beta) is stored in operand order: a 32 x 16 block is 64
@@ -176,24 +171,21 @@ constexpr int kRowXg = 0;                             // rk_i e^gamma_i [64]
 constexpr int kRowEg = kRowXg + kChunk;               // scale e^gamma_i [64]
 constexpr int kRowKs = kRowEg + kChunk;               // rk_i e^(gamma_C - gamma_i) [64]
 constexpr int kRowGl = kRowKs + kChunk;               // e^gamma_C [64 copies]
-constexpr int kRowGa = kRowGl + kChunk;               // gamma_i log2(e) [64]
-constexpr int kRowRk = kRowGa + kChunk;               // scale rk_i [64]
-constexpr int kScaleFloats = kRowRk + 3 * kChunk;     // padded to whole 1 KiB DMA pieces
+constexpr int kRowGa = kRowGl + kChunk;               // gamma_i log2(e) [64], hi
+constexpr int kRowGaLo = kRowGa + kChunk;             //   lo
+constexpr int kRowRk = kRowGaLo + kChunk;             // scale rk_i [64]
+constexpr int kScaleFloats = kRowRk + 2 * kChunk;     // padded to whole 1 KiB DMA pieces
 constexpr int kSlotFloats = kSlotScales + kScaleFloats;
 static_assert(kSlotScales % 256 == 0 && kScaleFloats % 256 == 0, "whole 1 KiB DMA pieces");
 static_assert(tri_blk(1, 3) == kTriBlocks - 1, "six lower blocks");
 
 // The combine's key order: first of the 4 keys that row tile t holds in lane
 // group g (items e = 0..3 are that key + e): tiles 2 kb and 2 kb + 1 together
-// are keys 32 kb + 8 g .. + 7, the key order of frag().  Row i of tile t is
+// are keys 32 kb + 8 g .. + 7, the combine's operand.  Row i of tile t is
 // thus key state_key(t, i / 4) + i % 4.
 __host__ __device__ constexpr int state_key(int t, int g) {
   return 32 * (t >> 1) + 8 * g + 4 * (t & 1);
 }
-
-// LDS row strides (elements) chosen so MFMA operand reads spread over banks.
-constexpr int kBfStride = kDim + 8;       // bf16 rows of 128
-constexpr int kF64Stride = kChunk + 4;    // fp32 rows of 64
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
   return __uint_as_float(static_cast<uint32_t>(h) << 16);
@@ -256,12 +248,6 @@ __device__ __forceinline__ s16x8 cat(s16x4 a, s16x4 b) {
   return s16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 }
 
-// Operand items of lane group g for key block kb of a bf16 row of 128 keys
-// in LDS: keys 32 kb + 8 g .. + 7, one 16-byte read (rows 16-byte aligned).
-__device__ __forceinline__ s16x8 frag(const uint16_t* row, int kb, int g) {
-  return *reinterpret_cast<const s16x8*>(row + 32 * kb + 8 * g);
-}
-
 struct Params {
   const uint16_t* q;         // [L, H, 128] bf16
   const uint16_t* k;         // [L, H, 128] bf16
@@ -302,7 +288,8 @@ struct Params {
   // most kFewSeqs sequences); if every sequence has at most this many tokens
   // it ran the whole prefill and these kernels return at once.
   int short_limit;
-  int prep_heads;            // v-heads per preparation workgroup: ratio, or 1
+  int prep_heads;            // v-heads per preparation wave: ratio, or 1
+  int prep_waves;            // waves per preparation workgroup: kPrepWaves, or 1
 };
 
 // Token range [start, end) of sequence s, clamped to [0, L] so that no
@@ -502,24 +489,28 @@ __device__ __forceinline__ void gates_of(uint16_t a_raw, uint16_t b_raw, float d
   beta = __builtin_amdgcn_rcpf(1.0f + __expf(-bf16_to_f32(b_raw)));
 }
 
-__device__ __forceinline__ void token_gates(const Params& p, int t, int hv, float& log2g,
-                                            float& beta) {
-  gates_of(p.a[static_cast<size_t>(t) * p.HV + hv], p.b[static_cast<size_t>(t) * p.HV + hv],
-           p.dt_bias[hv], p.A_log[hv], log2g, beta);
-}
-
 // One DPP step of a wave scan: x from the lane CTRL names (0 where it names
 // none, or in rows ROW_MASK leaves out).
 template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_add_src(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
-                                                               CTRL, ROW_MASK, 0xf, false));
+__device__ __forceinline__ double dpp_add_src(double x) {
+  const u32x2 w = __builtin_bit_cast(u32x2, x);
+  u32x2 r;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    r[i] = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(w[i]), CTRL,
+                                                             ROW_MASK, 0xf, false));
+  return __builtin_bit_cast(double, r);
 }
 
 // Inclusive prefix sum over the 64 lanes of a wave: shifts by 1, 2, 4 and 8
 // within each row of 16 lanes (row_shr), then lane 15's total added to rows
-// 1 and 3 and lane 31's to rows 2 and 3 (row_bcast:15, row_bcast:31).
-__device__ __forceinline__ float wave_prefix_sum(float x) {
+// 1 and 3 and lane 31's to rows 2 and 3 (row_bcast:15, row_bcast:31).  In 64
+// bits: a head that forgets fast reaches gamma ~ -1000 within a chunk, where
+// an fp32 sum is only good to 1e-4 and so are the decays e^(gamma_i - gamma_j)
+// of its last tokens; as hi + lo pairs the differences are good to 2^-24 of
+// themselves (state error against 64 bits on short sequences: up to 1.5e-5
+// with fp32 sums, 3-5e-6 -- the products' hi/lo splits -- with these).
+__device__ __forceinline__ double wave_prefix_sum(double x) {
   x += dpp_add_src<0x111, 0xf>(x);
   x += dpp_add_src<0x112, 0xf>(x);
   x += dpp_add_src<0x114, 0xf>(x);
@@ -529,328 +520,304 @@ __device__ __forceinline__ float wave_prefix_sum(float x) {
   return x;
 }
 
-// Rows [0, 64) of a [*, stride, 128] bf16 tensor (row r at base + r * step
-// elements) as 4 pieces of 16 bytes per thread.  Rows >= n read row n - 1
-// (n >= 1) so that every load is unconditional: issued together, waited on
-// once.  store_rows_bf16 writes them to LDS rows of kBfStride, zeroing rows
-// >= n.
-__device__ __forceinline__ void load_rows_bf16(u32x4 (&val)[4], const uint16_t* base,
-                                               size_t step, int n) {
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int idx = threadIdx.x + it * kThreads;
-    const int r = idx >> 4;
-    const int rr = r < n ? r : n - 1;
-    val[it] = *reinterpret_cast<const u32x4*>(base + static_cast<size_t>(rr) * step +
-                                              (idx & 15) * 8);
-  }
-}
-
-__device__ __forceinline__ void store_rows_bf16(uint16_t* dst, const u32x4 (&val)[4], int n) {
-#pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int idx = threadIdx.x + it * kThreads;
-    const int r = idx >> 4;
-    const u32x4 x = r < n ? val[it] : u32x4{0u, 0u, 0u, 0u};
-    uint16_t* d = dst + r * kBfStride + (idx & 15) * 8;
-    *reinterpret_cast<u32x2*>(d) = u32x2{x.x, x.y};
-    *reinterpret_cast<u32x2*>(d + 4) = u32x2{x.z, x.w};
-  }
+// 2^((xh + xl) - (yh + yl)), for x <= y; the clamp keeps what a mask discards
+// (x > y) finite.
+__device__ __forceinline__ float decay(float xh, float xl, float yh, float yl) {
+  return __builtin_amdgcn_exp2f(fminf((xh - yh) + (xl - yl), 0.0f));
 }
 
 // ---------------------------------------------------------------------------
 // 2. per-chunk preparation
 // ---------------------------------------------------------------------------
+// One wave per chunk and q/k head (its v-heads one after another) or v-head.
+// The chain of one chunk -- K K^T, gates, A, the triangular inverse by 16 x 16
+// blocks -- has little work in each step, so what bounds it is latency: four
+// waves sharing it waited 53% of their cycles on ten barriers and on LDS round
+// trips, 12 KiB of K rows and two 64 x 64 matrices there limited a CU to four
+// such chains, and each diagonal block's substitution used 16 of 64 lanes.  A
+// wave of its own needs no barrier, keeps K K^T's operands and every block in
+// registers in the two layouts the products read (6 KiB of LDS and 149
+// registers: twelve chains a CU), and runs the four substitutions at once.  Kernel
+// trace, before and after: 64 x 512 tokens at 16/32 heads 112-119 -> 82 us (4.5
+// TB/s of K rows in and slots out), 12 ragged sequences there 43 -> 28 us, 16 x
+// 1024 at 4/8 18.3 -> 14.6 us.
+//
+// 16 x 16 blocks in registers, lane (i, g) = (lane % 16, lane / 16), item e:
+//   column layout  [4 g + e][i]   (an MFMA result; the B operand)
+//   row layout     [i][4 g + e]   (the A operand)
+// with the contracted index taken as 4 g + (step) on both sides.  A result of
+// swapped operands is the product's transpose, i.e. the row layout:
+// (L X)^T = X^T L^T, where X's column layout reads as X^T's A operand and L's
+// row layout as L^T's B operand.
 
-// 35 KiB, so that four workgroups share a CU: A takes the place of the K
-// rows, which no wave reads once K K^T is in registers (every wave passes a
-// barrier between its last K read and the first write of A).  The 32 x 32
-// scratch of the block recursion is T's upper-right quarter, which T never
-// uses (rows 0..31, columns 32..63).
+constexpr int kPrepWaves = 4;       // a workgroup
+constexpr int kBlkStride = 20;      // floats of a 16-long row or column: 16-byte aligned,
+                                    // and reads down a column spread over the banks
+
 struct __attribute__((aligned(16))) PrepLds {
-  union {
-    uint16_t K[kChunk * kBfStride];   // the chunk's K rows, until K K^T
-    float A[kChunk * kF64Stride];     // then: strict lower part of (I + A) minus I
-  };
-  float T[kChunk * kF64Stride];       // (I + A)^-1
-  float gamma[kChunk];
+  float blk[4][16 * kBlkStride];    // the diagonal blocks of A by rows, then of T by columns
+  float gamma[kChunk];              // hi and lo
+  float gamma_lo[kChunk];
   float beta[kChunk];
   float rk[kChunk];
 };
-static_assert(sizeof(PrepLds) <= 160 * 1024 / 4, "four preparation workgroups per CU");
 
-// 16 x 16 x 16 fp32 block product A[0:16, 0:16] B[0:16, 0:16] from LDS rows
-// of stride lda / ldb, as an MFMA result (lane (col, g) holds rows 4 g + e).
-__device__ __forceinline__ f32x4 mm16_f32(const float* A, int lda, const float* B, int ldb,
-                                          int col, int g4) {
-  f32x4 acc = {0, 0, 0, 0};
+// A B (contracted over 16, fp32 MFMA) added to acc: rows of A in row layout,
+// B in column layout.
+__device__ __forceinline__ f32x4 mm16(const f32x4& a, const f32x4& b, f32x4 acc) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-    acc = mfma_f32(A[col * lda + 4 * ks + g4], B[(4 * ks + g4) * ldb + col], acc);
+  for (int ks = 0; ks < 4; ++ks) acc = mfma_f32(a[ks], b[ks], acc);
   return acc;
 }
 
-__device__ __forceinline__ void store16(float* D, int ldd, const f32x4& v, float sign, int col,
-                                        int g4) {
-#pragma unroll
-  for (int e = 0; e < 4; ++e) D[(4 * g4 + e) * ldd + col] = sign * v[e];
+__device__ __forceinline__ f32x4 lds4(const float* ptr) {
+  return *reinterpret_cast<const f32x4*>(ptr);
 }
 
 // One chunk's preparation, tokens t0 .. t0 + n - 1 (n: 1..64) of q/k head h,
-// for v-heads hv0 .. hv0 + prep_heads - 1, by the 256 threads of the calling
-// workgroup: the slots go to the workspace (slot c), or with LDS_SLOT (one
-// v-head) to lds_T and lds_scales in the calling workgroup's LDS.
+// for v-heads hv0 .. hv0 + prep_heads - 1, by the calling wave: the slots go
+// to the workspace (slot c), or with LDS_SLOT (one v-head) to lds_T and
+// lds_scales in the calling workgroup's LDS.
 template <bool LDS_SLOT>
-__device__ __forceinline__ void prep_chunk(Params p, int c, int t0, int n, int hv0, int h,
+__device__ __forceinline__ void prep_chunk(const Params& p, int c, int t0, int n, int hv0, int h,
                                            int prep_heads, PrepLds& lds, uint16_t* lds_T,
                                            float* lds_scales) {
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int col = lane & 15;
-  const int g4 = lane >> 4;
+  const int i = lane & 15;
+  const int g = lane >> 4;
+  const f32x4 zero = {0, 0, 0, 0};
 
-  // Every input load of the chunk is issued before the first is waited on.
-  u32x4 kreg[4];
-  load_rows_bf16(kreg, p.k + (static_cast<size_t>(t0) * p.H + h) * kDim,
-                 static_cast<size_t>(p.H) * kDim, n);
-  // wave 0's gate inputs (a, b of token t0 + lane) of the group's first
-  // kPrepGateHeads v-heads, in flight with the K rows
-  uint16_t a_raw[kPrepGateHeads], b_raw[kPrepGateHeads];
-  float dtb[kPrepGateHeads], alog[kPrepGateHeads];
-  if (wave == 0) {
-    const size_t tk = static_cast<size_t>(t0 + (lane < n ? lane : n - 1)) * p.HV + hv0;
-#pragma unroll
-    for (int j = 0; j < kPrepGateHeads; ++j) {
-      const int jj = j < prep_heads ? j : 0;
-      a_raw[j] = p.a[tk + jj];
-      b_raw[j] = p.b[tk + jj];
-      dtb[j] = p.dt_bias[hv0 + jj];
-      alog[j] = p.A_log[hv0 + jj];
-    }
-  }
-
-  store_rows_bf16(lds.K, kreg, n);
-  // T's upper blocks that the block recursion multiplies, T_01 and T_23, are
-  // zero; the diagonal and lower blocks are all written, the other upper
-  // blocks never read.
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const int idx = threadIdx.x + it * kThreads;
-    const int o = 32 * (idx >> 8);
-    lds.T[(o + ((idx >> 4) & 15)) * kF64Stride + o + 16 + (idx & 15)] = 0.0f;
-  }
-  block_sync_lds();
-
-  // K row scales of the L2-norm (1 when off): 4 threads per row.
+  // K K^T's lower blocks, in row layout: kk[r (r + 1) / 2 + cb] is rows 16 r
+  // + i, columns 16 cb + 4 g + e.  The operands (row 16 r + i, keys 32 m + 8 g
+  // .. + 7) come straight from memory, rows >= n as zeros; the first v-head's
+  // gate inputs are in flight with them.
+  const int tok = t0 + (lane < n ? lane : n - 1);
+  uint16_t a_raw = p.a[static_cast<size_t>(tok) * p.HV + hv0];
+  uint16_t b_raw = p.b[static_cast<size_t>(tok) * p.HV + hv0];
+  float dtb = p.dt_bias[hv0], alog = p.A_log[hv0];
+  f32x4 kk[10];
   {
-    const int r = threadIdx.x >> 2;
-    const int part = threadIdx.x & 3;
-    float sk = 0.0f;
-    if (p.l2norm) {
-      for (int i = part * 32; i < part * 32 + 32; ++i) {
-        const float y = bf16_to_f32(lds.K[r * kBfStride + i]);
-        sk = fmaf(y, y, sk);
-      }
-      sk += __shfl_xor(sk, 1, 64);
-      sk += __shfl_xor(sk, 2, 64);
+    s16x8 kf[4][4];
+    const uint16_t* base = p.k + (static_cast<size_t>(t0) * p.H + h) * kDim + 8 * g;
+    const size_t step = static_cast<size_t>(p.H) * kDim;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = min(16 * r + i, n - 1);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        kf[r][m] = *reinterpret_cast<const s16x8*>(base + row * step + 32 * m);
     }
-    if (part == 0) lds.rk[r] = p.l2norm ? __builtin_amdgcn_rsqf(sk + kL2Eps) : 1.0f;
-  }
-  block_sync_lds();
-
-  // K K^T for row block `wave` (rows 16 wave .. +15), column blocks 0 ..
-  // wave (A is strictly lower triangular: the blocks right of the diagonal
-  // are neither computed nor written); bf16 MFMA over the 128-long rows
-  f32x4 kk[4];
-  {
+    if (n < kChunk) {                                // uniform
 #pragma unroll
-    for (int nj = 0; nj < 4; ++nj) kk[nj] = f32x4{0, 0, 0, 0};
-    const int ra = wave * 16 + col;
+      for (int r = 0; r < 4; ++r)
 #pragma unroll
-    for (int m = 0; m < kDim / 32; ++m) {
-      const s16x8 ak = frag(&lds.K[ra * kBfStride], m, g4);
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj) {
-        if (nj > wave) break;                      // uniform per wave
-        const s16x8 bk = frag(&lds.K[(nj * 16 + col) * kBfStride], m, g4);
-        kk[nj] = mfma_bf16(ak, bk, kk[nj]);
-      }
+        for (int m = 0; m < 4; ++m)
+          if (16 * r + i >= n) kf[r][m] = s16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int cb = 0; cb <= r; ++cb) {
+        f32x4 acc = zero;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc = mfma_bf16(kf[cb][m], kf[r][m], acc);
+        kk[r * (r + 1) / 2 + cb] = acc;
+      }
   }
 
-  // Each v-head of the group: its gates, A from the shared product, T, and
-  // its slot.  The LDS the previous v-head used (gamma, beta, A, T)
-  // is rewritten only after the barrier that ends its use.
+  // K row scales of the L2-norm (1 when off), |k|^2 from K K^T's diagonal
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const f32x4 d = kk[r * (r + 1) / 2 + r];
+    const float k2 = (i & 2) ? ((i & 1) ? d[3] : d[2]) : ((i & 1) ? d[1] : d[0]);
+    if (g == (i >> 2)) lds.rk[16 * r + i] = p.l2norm ? __builtin_amdgcn_rsqf(k2 + kL2Eps) : 1.0f;
+  }
+
   for (int j = 0; j < prep_heads; ++j) {
     const int hv = hv0 + j;
     float* const slot = LDS_SLOT ? nullptr
                                  : p.slots + (static_cast<size_t>(c) * p.HV + hv) * kSlotFloats;
     uint16_t* const T16 = LDS_SLOT ? lds_T : reinterpret_cast<uint16_t*>(slot);
     float* const scales = LDS_SLOT ? lds_scales : slot + kSlotScales;
+
     // gates of token t0 + lane (padded rows: no decay, no update), and the
     // inclusive scan of the log-decay over the chunk
-    if (wave == 0) {
-      float log2g, beta;
-      if (j < kPrepGateHeads) {
-        uint16_t ar = a_raw[0], br = b_raw[0];
-        float dt = dtb[0], al = alog[0];
-#pragma unroll
-        for (int jj = 1; jj < kPrepGateHeads; ++jj)
-          if (j == jj) { ar = a_raw[jj]; br = b_raw[jj]; dt = dtb[jj]; al = alog[jj]; }
-        gates_of(ar, br, dt, al, log2g, beta);
-      } else {
-        token_gates(p, t0 + (lane < n ? lane : n - 1), hv, log2g, beta);
-      }
-      if (lane >= n) log2g = beta = 0.0f;
-      lds.gamma[lane] = wave_prefix_sum(log2g);
-      lds.beta[lane] = beta;
+    float log2g, beta;
+    gates_of(a_raw, b_raw, dtb, alog, log2g, beta);
+    if (j + 1 < prep_heads) {                        // the next v-head's inputs
+      a_raw = p.a[static_cast<size_t>(tok) * p.HV + hv + 1];
+      b_raw = p.b[static_cast<size_t>(tok) * p.HV + hv + 1];
+      dtb = p.dt_bias[hv + 1];
+      alog = p.A_log[hv + 1];
     }
-    block_sync_lds();
-    {
-      // Row and column factors, read once.  The decays are computed for every
-      // element with the exponent clamped to <= 0 (it is <= 0 wherever the
-      // element is kept: gamma does not increase) and the masks are selects.
-      // A[i][j], i = 16 wave + 4 g + e, j = 16 nj + col (K K^T is symmetric)
-      const int ia = wave * 16 + g4 * 4;
-      const f32x4 gi4 = *reinterpret_cast<const f32x4*>(&lds.gamma[ia]);
-      const f32x4 bri4 = *reinterpret_cast<const f32x4*>(&lds.beta[ia]) *
-                         *reinterpret_cast<const f32x4*>(&lds.rk[ia]);
+    if (lane >= n) log2g = beta = 0.0f;
+    const double gamma64 = wave_prefix_sum(static_cast<double>(log2g));
+    const float gamma = static_cast<float>(gamma64);
+    const float gamma_lo = static_cast<float>(gamma64 - static_cast<double>(gamma));
+    __builtin_amdgcn_wave_barrier();
+    lds.gamma[lane] = gamma;
+    lds.gamma_lo[lane] = gamma_lo;
+    lds.beta[lane] = beta;
+    __builtin_amdgcn_wave_barrier();
+
+    // A's blocks below the diagonal, row layout; the diagonal ones (strictly
+    // lower) by rows to LDS.  The decays are computed for every element with
+    // the exponent clamped to <= 0 (it is <= 0 wherever the element is kept:
+    // gamma does not increase) and the masks are selects.
+    f32x4 gj[4], gjl[4], rkj[4];
 #pragma unroll
-      for (int nj = 0; nj < 4; ++nj) {
-        if (nj > wave) break;                      // uniform: never read
-        const int j = nj * 16 + col;
-        const float gj = lds.gamma[j];
-        const float rkj = lds.rk[j];
+    for (int cb = 0; cb < 4; ++cb) {
+      gj[cb] = lds4(&lds.gamma[16 * cb + 4 * g]);
+      gjl[cb] = lds4(&lds.gamma_lo[16 * cb + 4 * g]);
+      rkj[cb] = lds4(&lds.rk[16 * cb + 4 * g]);
+    }
+    f32x4 A[10];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float gi = lds.gamma[16 * r + i], gil = lds.gamma_lo[16 * r + i];
+      const float bri = lds.beta[16 * r + i] * lds.rk[16 * r + i];
+#pragma unroll
+      for (int cb = 0; cb <= r; ++cb) {
+        const int at = r * (r + 1) / 2 + cb;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float dec = __builtin_amdgcn_exp2f(fminf(gi4[e] - gj, 0.0f));
-          const float x = bri4[e] * rkj * dec * kk[nj][e];
-          lds.A[(ia + e) * kF64Stride + j] = j < ia + e ? x : 0.0f;
+          const float dec = decay(gi, gil, gj[cb][e], gjl[cb][e]);
+          const float x = bri * rkj[cb][e] * dec * kk[at][e];
+          A[at][e] = cb < r || 4 * g + e < i ? x : 0.0f;
         }
       }
+      *reinterpret_cast<f32x4*>(&lds.blk[r][i * kBlkStride + 4 * g]) = A[r * (r + 1) / 2 + r];
     }
-    block_sync_lds();
+    __builtin_amdgcn_wave_barrier();
 
     // T = (I + A)^-1 by block recursion on 16 x 16 blocks (A is strictly lower
-    // triangular, so T is unit lower triangular; the upper blocks stay zero):
-    // 1. each wave inverts one diagonal block by forward substitution (one
-    //    column per lane, two partial sums per dot product);
-    //    Row r's entries of A are read as 16-byte vectors a row ahead of
-    //    their use (read when used, their LDS latency was most of the
-    //    substitution's).
-    if (lane < 16) {
-      const int b0 = wave * 16;
-      const float* arow = &lds.A[b0 * kF64Stride + b0];
+    // triangular, so T is unit lower triangular):
+    // 1. lane (i, g) solves for column i of diagonal block g by forward
+    //    substitution, two partial sums per dot product; row r's entries of A
+    //    are read a row ahead of their use;
+    f32x4 TD[4], TR[4];                              // column, row layout
+    {
+      const float* arow = lds.blk[g];
       float t[16];
       f32x4 ar[16][4];
       auto read_row = [&](int r) {
 #pragma unroll
-        for (int q = 0; q < (r + 3) / 4; ++q)
-          ar[r][q] = *reinterpret_cast<const f32x4*>(&arow[r * kF64Stride + 4 * q]);
+        for (int q = 0; q < (r + 3) / 4; ++q) ar[r][q] = lds4(&arow[r * kBlkStride + 4 * q]);
       };
       read_row(1);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         if (r + 1 < 16) read_row(r + 1);
-        float s0 = (r == lane) ? 1.0f : 0.0f, s1 = 0.0f;
+        float s0 = (r == i) ? 1.0f : 0.0f, s1 = 0.0f;
 #pragma unroll
-        for (int j = 0; j < r; ++j) {
-          const float aij = ar[r][j >> 2][j & 3];
-          if (j & 1) s1 = fmaf(-aij, t[j], s1); else s0 = fmaf(-aij, t[j], s0);
+        for (int q = 0; q < r; ++q) {
+          const float aij = ar[r][q >> 2][q & 3];
+          if (q & 1) s1 = fmaf(-aij, t[q], s1); else s0 = fmaf(-aij, t[q], s0);
         }
         t[r] = s0 + s1;
-        lds.T[(b0 + r) * kF64Stride + b0 + lane] = t[r];
       }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<f32x4*>(&lds.blk[g][i * kBlkStride + 4 * q]) =
+            f32x4{t[4 * q], t[4 * q + 1], t[4 * q + 2], t[4 * q + 3]};
+      __builtin_amdgcn_wave_barrier();
     }
-    block_sync_lds();
-    // 2. the 32 x 32 diagonal halves: T_10 = -T_11 A_10 T_00 (wave 0) and
-    //    T_32 = -T_33 A_32 T_22 (wave 1), through LDS within the wave;
-    if (wave < 2) {
-      const int b = wave * 32;
-      float* Xw = &lds.T[32] + wave * 16 * kF64Stride;
-      const f32x4 x = mm16_f32(&lds.A[(b + 16) * kF64Stride + b], kF64Stride,
-                               &lds.T[b * kF64Stride + b], kF64Stride, col, g4);
-      store16(Xw, kF64Stride, x, 1.0f, col, g4);
-      const f32x4 y = mm16_f32(&lds.T[(b + 16) * kF64Stride + b + 16], kF64Stride, Xw,
-                               kF64Stride, col, g4);
-      store16(&lds.T[(b + 16) * kF64Stride + b], kF64Stride, y, -1.0f, col, g4);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      TD[b] = lds4(&lds.blk[b][i * kBlkStride + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) TR[b][e] = lds.blk[b][(4 * g + e) * kBlkStride + i];
     }
-    block_sync_lds();
-    // 3. the lower-left 32 x 32 quarter: T_BA = -T_B (A_BA T_A), one 16 x 16
-    //    tile per wave.
-    {
-      const int rb = wave >> 1, cb = wave & 1;
-      const float* Arow = &lds.A[(32 + 16 * rb) * kF64Stride];
-      const f32x4 x = mm16_f32(Arow, kF64Stride, &lds.T[16 * cb], kF64Stride, col, g4) +
-                      mm16_f32(Arow + 16, kF64Stride, &lds.T[16 * kF64Stride + 16 * cb],
-                               kF64Stride, col, g4);
-      store16(&lds.T[16 * rb * kF64Stride + 32 + 16 * cb], kF64Stride, x, 1.0f, col, g4);
+    // 2. the 32 x 32 diagonal halves: T_10 = -T_11 A_10 T_00, T_32 = -T_33
+    //    A_32 T_22;
+    const f32x4 x10 = mm16(A[1], TD[0], zero);
+    const f32x4 x32 = mm16(A[8], TD[2], zero);
+    const f32x4 T10D = -mm16(TR[1], x10, zero);
+    const f32x4 T10 = -mm16(x10, TR[1], zero);
+    const f32x4 T32 = -mm16(x32, TR[3], zero);
+    // 3. the lower-left 32 x 32 quarter: T_BA = -T_B (A_BA T_A).
+    f32x4 T[10];                                     // row layout, as A
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb) {
+      f32x4 x[2];
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb) {
+        const int at = (2 + rb) * (3 + rb) / 2;
+        x[rb] = cb == 0 ? mm16(A[at + 1], T10D, mm16(A[at], TD[0], zero))
+                        : mm16(A[at + 1], TD[1], zero);
+      }
+      T[3 + cb] = -mm16(x[0], TR[2], zero);
+      T[6 + cb] = -mm16(x[1], TR[3], mm16(x[0], T32, zero));
     }
-    block_sync_lds();
-    {
-      const int rb = wave >> 1, cb = wave & 1;
-      const float* Trow = &lds.T[(32 + 16 * rb) * kF64Stride + 32];
-      const float* X = &lds.T[32];
-      const f32x4 y = mm16_f32(Trow, kF64Stride, &X[16 * cb], kF64Stride, col, g4) +
-                      mm16_f32(Trow + 16, kF64Stride, &X[16 * kF64Stride + 16 * cb], kF64Stride,
-                               col, g4);
-      store16(&lds.T[(32 + 16 * rb) * kF64Stride + 16 * cb], kF64Stride, y, -1.0f, col, g4);
-    }
-    block_sync_lds();
+    T[0] = TR[0];
+    T[1] = T10;
+    T[2] = TR[1];
+    T[5] = TR[2];
+    T[8] = T32;
+    T[9] = TR[3];
 
-    // T diag(beta) in operand order: lower block (rb, kb) holds, for lane
-    // (m, g), T[32 rb + m][16 kb + k] beta[16 kb + k] at the 8 k of its items
-    // (4 g .. + 3 and 8 + 4 g .. + 3).  Wave w writes block w, waves 0 and 1
-    // also blocks 4 and 5.  Blocks (0, 1) and (1, 3) read T_01 and T_23
-    // (zero); none reads the recursion's scratch quarter.
+    // T diag(beta) in operand order, split into hi + lo: row 16 r + i, tokens
+    // 16 cb + 4 g .. + 3 are items 4 (g / 2) .. + 3 of lane 16 (r % 2) + i +
+    // 32 (g % 2) of block (r / 2, cb).  Blocks (0, 1) and (2, 3), above the
+    // diagonal inside an operand block, are zero.
+    uint16_t* const dst0 = T16 + (i + 32 * (g & 1)) * 8 + 4 * (g >> 1);
 #pragma unroll
-    for (int rep = 0; rep < 2; ++rep) {
-      const int idx = wave + 4 * rep;
-      if (idx >= kTriBlocks) break;                  // uniform per wave
-      const int rb = idx < 2 ? 0 : 1, kb = idx - 2 * rb;     // tri_blk(rb, kb) == idx
-      const int g2 = lane >> 5;
-      const float* trow = &lds.T[(32 * rb + (lane & 31)) * kF64Stride + 16 * kb + 4 * g2];
-      const float* brow = &lds.beta[16 * kb + 4 * g2];
-      s16x4 hi[2], lo[2];
+    for (int r = 0; r < 4; ++r) {
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
-        split4(*reinterpret_cast<const f32x4*>(trow + 8 * hf) *
-                   *reinterpret_cast<const f32x4*>(brow + 8 * hf),
-               hi[hf], lo[hf]);
-      uint16_t* const dst = T16 + idx * kBlk + lane * 8;
-      *reinterpret_cast<s16x8*>(dst) = cat(hi[0], hi[1]);
-      *reinterpret_cast<s16x8*>(dst + kTriBlocks * kBlk) = cat(lo[0], lo[1]);
+      for (int cb = 0; cb <= (r | 1); ++cb) {
+        s16x4 hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
+        if (cb <= r) split4(T[r * (r + 1) / 2 + cb] * lds4(&lds.beta[16 * cb + 4 * g]), hi, lo);
+        uint16_t* const dst = dst0 + tri_blk(r >> 1, cb) * kBlk + 128 * (r & 1);
+        *reinterpret_cast<s16x4*>(dst) = hi;
+        *reinterpret_cast<s16x4*>(dst + kTriBlocks * kBlk) = lo;
+      }
     }
 
     // Row scales for the scan: the decayed K rows of X, the decay of the
     // output's rows (times the scale), the K rows of the state update, the
     // chunk decay, and gamma and the K row scales (times the scale) for its P.
-    if (wave == 1) {
-      const float gl = lds.gamma[kChunk - 1];        // padded rows carry gamma forward
-      const float gi = lds.gamma[lane];
+    {
+      // padded rows carry gamma forward
+      auto last = [](float x) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), kChunk - 1));
+      };
       const float rki = lds.rk[lane];
-      const float egi = __builtin_amdgcn_exp2f(gi);
+      const float e0 = __builtin_amdgcn_exp2f(gamma);
+      const float egi = fmaf(e0, gamma_lo * kLn2, e0);
       scales[kRowXg + lane] = rki * egi;
       scales[kRowEg + lane] = p.scale * egi;
-      scales[kRowKs + lane] = rki * __builtin_amdgcn_exp2f(gl - gi);
-      scales[kRowGl + lane] = __builtin_amdgcn_exp2f(gl);
-      scales[kRowGa + lane] = gi;
+      scales[kRowKs + lane] = rki * decay(last(gamma), last(gamma_lo), gamma, gamma_lo);
+      scales[kRowGl + lane] = last(egi);
+      scales[kRowGa + lane] = gamma;
+      scales[kRowGaLo + lane] = gamma_lo;
       scales[kRowRk + lane] = p.scale * rki;
     }
-    block_sync_lds();                        // this v-head's LDS reads are done
   }
 }
 
 // FEW: the batch's chunk slots come from cu_seqlens in the kernel (few
 // sequences, no offsets kernel); a template flag, so that the kernels of the
 // other modes are compiled without that code.
+// Four independent waves a workgroup: four jobs (v-head groups, or v-heads) of
+// one slot, whose K rows they share, or with fewer jobs a slot one job of four
+// slots.  With at most four waves a CU in all, one wave a workgroup, so that
+// they spread over the CUs (160 jobs, 4 ragged sequences at 4/8 heads: 9.4 ->
+// 7.3 us; 2176 jobs, 16 x 1024 tokens there: 15.5 us so, 14.6 us by four).
 template <bool FEW>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(64 * kPrepWaves) __attribute__((amdgpu_waves_per_eu(3)))
 void prep_kernel(Params p) {
-  __shared__ PrepLds lds;
-  const int c = blockIdx.x;
+  __shared__ PrepLds lds_all[kPrepWaves];
+  const int wave = wave_index();
+  const int jobs = p.HV / p.prep_heads;
+  const bool by_job = jobs >= p.prep_waves;
+  const long long c64 = by_job ? static_cast<long long>(blockIdx.x)
+                               : static_cast<long long>(blockIdx.x) * p.prep_waves + wave;
+  const int job = static_cast<int>(by_job ? blockIdx.y * p.prep_waves + wave : blockIdx.y);
+  if (c64 >= p.max_slots || job >= jobs) return;   // uniform per wave; no barriers below
+  const int c = static_cast<int>(c64);
   // v-heads hv0 .. hv0 + prep_heads - 1, all of q/k head h
-  const int hv0 = static_cast<int>(blockIdx.y) * p.prep_heads;
+  const int hv0 = job * p.prep_heads;
   const int h = hv0 / p.ratio;
   if (p.short_limit > 0 && all_within(p, p.short_limit)) return;    // uniform
   int t0, n;                                       // n: 1..64, 0 past the last slot
@@ -876,8 +843,10 @@ void prep_kernel(Params p) {
     t0 = info.y;
     n = info.z;
   }
-  if (n <= 0) return;                              // uniform per workgroup
-  prep_chunk<false>(p, c, t0, n, hv0, h, p.prep_heads, lds, nullptr, nullptr);
+  t0 = uniform(t0);
+  n = uniform(n);
+  if (n <= 0) return;                              // uniform per wave
+  prep_chunk<false>(p, c, t0, n, hv0, h, p.prep_heads, lds_all[wave], nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1143,14 +1112,15 @@ __device__ __forceinline__ void p_tile_ops(const uint16_t* Kr, const uint16_t* Q
 __device__ __forceinline__ void p_tile_store(const f32x4& acc, const ScanScales* Sc, PTile pt,
                                              int lane, uint16_t* Pb) {
   const int c = lane & 15, g4 = lane >> 4;
-  const float gi = Sc->row[kRowGa + 16 * pt.it + c];
-  const f32x4 gj = *reinterpret_cast<const f32x4*>(&Sc->row[kRowGa + 16 * pt.jt + 4 * g4]);
-  const f32x4 rkj = *reinterpret_cast<const f32x4*>(&Sc->row[kRowRk + 16 * pt.jt + 4 * g4]);
+  const float gi = Sc->row[kRowGa + 16 * pt.it + c], gil = Sc->row[kRowGaLo + 16 * pt.it + c];
+  const f32x4 gj = lds4(&Sc->row[kRowGa + 16 * pt.jt + 4 * g4]);
+  const f32x4 gjl = lds4(&Sc->row[kRowGaLo + 16 * pt.jt + 4 * g4]);
+  const f32x4 rkj = lds4(&Sc->row[kRowRk + 16 * pt.jt + 4 * g4]);
   const int lim = 16 * (pt.it - pt.jt) + c - 4 * g4;          // j <= i: e <= lim
   f32x4 pv;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const float y = rkj[e] * __builtin_amdgcn_exp2f(fminf(gi - gj[e], 0.0f)) * acc[e];
+    const float y = rkj[e] * decay(gi, gil, gj[e], gjl[e]) * acc[e];
     pv[e] = e <= lim ? y : 0.0f;
   }
   s16x4 hi, lo;
@@ -1706,8 +1676,9 @@ __device__ __forceinline__ void scan_body(Params p) {
 #pragma unroll
     for (int part = 0; part < 4; ++part)
       issue_part<OUT, false>(&In0, &S0, cx, first_src, part, wave, lane);
-    prep_chunk<true>(p, 0, start, end - start, hv, h, 1, *reinterpret_cast<PrepLds*>(&In1), In0.T,
-                     S0.row);
+    if (wave == 0)                                                             // uniform
+      prep_chunk<true>(p, 0, start, end - start, hv, h, 1, *reinterpret_cast<PrepLds*>(&In1),
+                       In0.T, S0.row);
     wait_vmem();
     block_sync_lds();
     side_tiles<OUT, L2>(&In0, &S0, Kt, Pb, Qn, Sel, wave, lane);
@@ -2123,6 +2094,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
   p.max_slots = slots;
   p.short_limit = maybe_all_short(total_seq_len, num_seqs) ? kSmallTokens : 0;
   p.prep_heads = prep_split(slots, HV) ? 1 : p.ratio;
+  p.prep_waves = slots * (HV / p.prep_heads) <= kPrepSpreadMaxWaves ? 1 : kPrepWaves;
 
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
   // events[i] (optional) is recorded before launch i and events[3] after the last
@@ -2179,8 +2151,11 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
   if (e != hipSuccess) return e;
   if (slots > 0) {
     auto* prep = p.few ? prep_kernel<true> : prep_kernel<false>;
-    hipLaunchKernelGGL(prep, dim3(static_cast<unsigned>(slots), HV / p.prep_heads),
-                       dim3(kThreads), 0, stream, p);
+    const int jobs = HV / p.prep_heads;
+    const int w = p.prep_waves;
+    const dim3 grid = jobs >= w ? dim3(static_cast<unsigned>(slots), (jobs + w - 1) / w)
+                                : dim3(static_cast<unsigned>((slots + w - 1) / w), jobs);
+    hipLaunchKernelGGL(prep, grid, dim3(64 * w), 0, stream, p);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

@@ -702,3 +702,38 @@ def test_one_chunk_kernel_matches_the_chunkwise_kernels_bitwise(l2, hip_device):
     out_1, st_1 = gdn.prefill_run(**_dev(alone, hip_device), use_qk_l2norm=l2)
     torch.cuda.synchronize()
     assert torch.equal(out_1, out_c[:64]) and torch.equal(st_1, st_c[:1])
+
+
+@pytest.mark.parametrize("lens,H,HV", [
+    ([5] * 1024 + [70], 1, 4),        # one job a slot: four slots a workgroup, the last three
+    ([6] * 341 + [130], 3, 12),       # three jobs a slot, v-heads of a group in turn
+    ([1, 16, 17, 33, 48, 49, 63], 5, 5),  # chunks that end in each 16-token block; five jobs
+])
+def test_preparation_jobs_at_their_edges(lens, H, HV, hip_device):
+    """The preparation's waves by job (a slot's v-head groups or v-heads) and
+    by slot, with jobs that do not fill the last workgroup."""
+    _announce(f"preparation jobs N={len(lens)} H={H} HV={HV}")
+    t = make_prefill_inputs(lens, H, HV, seed=500 + len(lens) + H)
+    out, st = gdn.prefill_run(**_dev(t, hip_device))
+    torch.cuda.synchronize()
+    _check(t, out, st, loop=False)
+
+
+@pytest.mark.parametrize("lens,l2", [([64], False), ([65, 128], True), ([300], True)])
+def test_fast_forgetting_heads_keep_the_split_precision(lens, l2, hip_device):
+    """Heads whose log-decay reaches -1000 within a chunk: the state's error
+    against float64 stays at that of the bf16 hi + lo operands (2^-17 of a
+    value each; 3e-6 in relative Frobenius norm measured), under 2^-16.  A
+    cumulative decay summed in fp32 is only good to 2^-24 of -1000 there, up
+    to 6e-5 on the last tokens' weights."""
+    _announce(f"fast-forgetting heads lens={lens} l2={l2}")
+    H, HV = 4, 8
+    t = make_prefill_inputs(lens, H, HV, seed=520 + sum(lens), unit_qk=not l2)
+    t["A_log"] = torch.log(torch.linspace(12.0, 16.0, HV))
+    t["dt_bias"] = torch.full((HV,), 1.5)
+    out, st = gdn.prefill_run(**_dev(t, hip_device), use_qk_l2norm=l2)
+    torch.cuda.synchronize()
+    _check(t, out, st, l2=l2, loop=False)
+    _, s64 = prefill_chunked_fp64(**t, use_qk_l2norm=l2)
+    err = np.linalg.norm(st.cpu().double().numpy() - s64) / np.linalg.norm(s64)
+    assert err < 2.0 ** -16, err
