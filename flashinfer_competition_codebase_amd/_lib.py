@@ -134,6 +134,34 @@ def get_prefill_lib() -> ctypes.CDLL:
     return _prefill_lib
 
 
+# The native call path of the entry points (``_gdn_host``, csrc/host.cpp), once
+# bound to both libraries by the first call that passed the Python checks.
+bound_host = None
+
+
+def bind_host() -> None:
+    """Load the native host module and bind it (once)."""
+    global bound_host
+    if bound_host is not None:
+        return
+    decode, prefill = get_lib(), get_prefill_lib()
+    try:
+        from . import _gdn_host as module
+    except ImportError as exc:
+        raise RuntimeError(f"native host module not loadable ({exc}); build it with "
+                           "`python -m flashinfer_competition_codebase_amd.build`") from exc
+
+    def address(fn):
+        return ctypes.cast(fn, ctypes.c_void_p).value
+
+    with _lock:
+        module.bind_decode(address(decode.gdn_decode_steps))
+        module.bind_prefill(address(prefill.gdn_prefill), address(prefill.gdn_prefill_noalloc),
+                            address(prefill.gdn_prefill_workspace_bytes),
+                            address(prefill.gdn_prefill_dispatches))
+        bound_host = module
+
+
 _raw_stream = None
 
 

@@ -10,7 +10,10 @@ this file:
   prefill (declared in ``include/gdn_prefill.h``);
 * ``csrc/calib.hip`` into ``libgdn_calib.so``: reference kernels (same-bytes
   read-modify-write, empty kernel) that only ``bench.py`` loads, to report
-  the floor of the decode step's traffic.
+  the floor of the decode step's traffic;
+* ``csrc/host.cpp`` into ``_gdn_host.so``: the entry points' checks,
+  allocations and call in native code (a CPython extension module against
+  the installed torch; host code only, compiled with g++).
 """
 
 from __future__ import annotations
@@ -31,6 +34,8 @@ CALIB_SRC = PKG_DIR / "csrc" / "calib.hip"
 CALIB_PATH = PKG_DIR / "libgdn_calib.so"
 PREFILL_SRC = PKG_DIR / "csrc" / "gdn_prefill.hip"
 PREFILL_PATH = PKG_DIR / "libgdn_prefill.so"
+HOST_SRC = PKG_DIR / "csrc" / "host.cpp"
+HOST_PATH = PKG_DIR / "_gdn_host.so"
 # library -> source
 LIBRARIES = {LIB_PATH: CSRC, PREFILL_PATH: PREFILL_SRC, CALIB_PATH: CALIB_SRC}
 OFFLOAD_ARCH = "gfx950"
@@ -97,13 +102,31 @@ def compile_command(out: Path = LIB_PATH, src: Path = CSRC,
     ]
 
 
+def host_compile_command(out: Path = HOST_PATH, src: Path = HOST_SRC) -> list[str]:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[f"-isystem{p}" for p in cpp_extension.include_paths()],
+            f"-isystem{sysconfig.get_paths()['include']}", f"-isystem{rocm}/include",
+            f"-I{INCLUDE_DIR}",
+            str(src), "-o", str(out),
+            f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10_hip", "-lc10"]
+
+
 def build(verbose: bool = False) -> Path:
     """Compile every library (always, even when built copies exist), in
     parallel; returns the decode library's path."""
     jobs = []
-    for lib, src in LIBRARIES.items():
+    for lib, src in {**LIBRARIES, HOST_PATH: HOST_SRC}.items():
         tmp = lib.with_suffix(".so.tmp")
-        cmd = compile_command(tmp, src, EXTRA_FLAGS.get(lib))
+        cmd = (host_compile_command(tmp, src) if lib == HOST_PATH
+               else compile_command(tmp, src, EXTRA_FLAGS.get(lib)))
         if verbose:
             print(" ".join(cmd), flush=True)
         jobs.append((lib, tmp, subprocess.Popen(cmd, stdout=subprocess.PIPE,
@@ -117,7 +140,7 @@ def build(verbose: bool = False) -> Path:
         else:
             os.replace(tmp, lib)
     if failed:
-        raise RuntimeError("hipcc failed: " + ", ".join(failed))
+        raise RuntimeError("compilation failed: " + ", ".join(failed))
     return LIB_PATH
 
 

@@ -357,20 +357,34 @@ def kernel_hip_shaped(q, k, v, state, A_log, a, dt_bias, b, scale, output,
     return None
 
 
-@torch.no_grad()
 def run(q, k, v, state, A_log, a, dt_bias, b, scale, *, use_qk_l2norm: bool = False):
     """Value-returning decode step with the reference's contract
     (``kernel_pt_reference``, solution/triton/kernel.py:22-118).
 
     Returns ``(output [B, T, HV, 128] bf16, new_state [B, HV, 128, 128])``,
     the new state in the state's dtype (fp32 for ``state=None``); ``state``
-    is not modified.
+    is not modified.  The checks, allocations and call run natively
+    (csrc/host.cpp); calls that path does not take run here.
     """
+    host = _lib.bound_host
+    if host is not None:
+        done = host.decode_run(q, k, v, state, A_log, a, dt_bias, b, scale, use_qk_l2norm)
+        if done is not None:
+            code, output, new_state = done
+            if code:
+                _lib.check(code, "gdn_decode_steps")
+            return output, new_state
+    return _run_checked(q, k, v, state, A_log, a, dt_bias, b, scale, use_qk_l2norm)
+
+
+@torch.no_grad()
+def _run_checked(q, k, v, state, A_log, a, dt_bias, b, scale, use_qk_l2norm):
     B, T, H, HV = check_inputs(q, k, v, state, A_log, a, dt_bias, b)
     sdtype = torch.float32 if state is None else state.dtype
     output = torch.empty((B, T, HV, V_DIM), dtype=torch.bfloat16, device=q.device)
     new_state = torch.empty((B, HV, V_DIM, K_DIM), dtype=sdtype, device=q.device)
     if B > 0:
+        _lib.bind_host()               # calls like this one run natively from here on
         # fresh outputs every call: launched directly, not bound for reuse
         _launch(q, k, v, state, A_log, a, dt_bias, b, resolve_scale(scale, q.shape[-1]),
                 output, new_state, B, T, H, HV, use_qk_l2norm)

@@ -118,12 +118,28 @@ def check_prefill_inputs(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, outpu
     return L, N, H, HV
 
 
-@torch.no_grad()
 def kernel_prefill_hip(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output,
                        new_state, *, use_qk_l2norm: bool = False):
     """Destination-passing prefill (reference DPS form,
     solution/triton/prefill_kernel.py:10-58): writes ``output`` and
-    ``new_state``; ``new_state is state`` updates in place."""
+    ``new_state``; ``new_state is state`` updates in place.  The checks and the
+    call run natively (csrc/host.cpp); calls that path does not take (errors,
+    conversions, another device current) run here."""
+    host = _lib.bound_host
+    if host is not None and output is not None and new_state is not None:
+        code = host.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output,
+                            new_state, use_qk_l2norm)
+        if code is not None:
+            if code:
+                _lib.check(code, "gdn_prefill")
+            return None
+    return _prefill_checked(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output,
+                            new_state, use_qk_l2norm)
+
+
+@torch.no_grad()
+def _prefill_checked(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_state,
+                     use_qk_l2norm):
     _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_state,
             use_qk_l2norm, None)
 
@@ -184,6 +200,7 @@ def _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new
         return None
     if cu_seqlens.dtype != torch.int32:
         cu_seqlens = cu_seqlens.to(torch.int32)
+    _lib.bind_host()                   # calls like this one run natively from here on
     lib = _lib.get_prefill_lib()
     ws_bytes = workspace_bytes(L, N, H, HV)
     workspace = torch.empty(ws_bytes + 256, dtype=torch.uint8, device=q.device)
@@ -210,7 +227,6 @@ def _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new
     return None
 
 
-@torch.no_grad()
 def prefill_run(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, *,
                 use_qk_l2norm: bool = False):
     """Value-returning prefill with the reference's contract
@@ -219,9 +235,24 @@ def prefill_run(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, *,
     ``state`` is not modified.  Tokens that no sequence covers (all of them
     when N = 0, those past ``cu_seqlens[N]`` otherwise) get zero outputs, as
     the reference's zero-initialised result (prefill_kernel.py:135-137)."""
+    host = _lib.bound_host
+    if host is not None:
+        done = host.prefill(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, None, None,
+                            use_qk_l2norm)
+        if done is not None:
+            code, output, new_state = done
+            if code:
+                _lib.check(code, "gdn_prefill")
+            return output, new_state
+    return _prefill_run_checked(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale,
+                                use_qk_l2norm)
+
+
+@torch.no_grad()
+def _prefill_run_checked(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, use_qk_l2norm):
     L, N, H, HV = check_prefill_inputs(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens)
     output = torch.zeros((L, HV, V_DIM), dtype=torch.bfloat16, device=q.device)
     new_state = torch.empty((N, HV, V_DIM, K_DIM), dtype=torch.float32, device=q.device)
-    kernel_prefill_hip(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output,
-                       new_state, use_qk_l2norm=use_qk_l2norm)
+    _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new_state,
+            use_qk_l2norm, None)
     return output, new_state
