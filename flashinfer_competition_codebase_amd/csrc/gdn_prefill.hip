@@ -1251,12 +1251,6 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
   const int m = lane & 31;
   const int g = lane >> 5;
 
-  // read ~3 k cycles ahead of their use (a chunk ahead, they hold registers
-  // through the second half, where the most are live)
-  u32x4 vf[4];
-  load_v(vf, cx, chunk_src(cx, ci), lane);
-  __builtin_amdgcn_sched_barrier(0);           // issued here, not before their use
-
   // piece 2 b + g of row 32 R + m, at position (2 b + g) ^ (m % 16)
   const unsigned row0 = static_cast<unsigned>(m) * kDim + 8u * (g ^ (m & 15));
   auto k_op = [&](int b, int R) { return ld_op(&In->Kr[(row0 ^ (16u * b)) + R * 32 * kDim]); };
@@ -1276,6 +1270,12 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
     }
   };
   read_ops(0, 0);
+  // V, ~3 k cycles ahead of its use (a chunk ahead, it holds registers through
+  // the second half, where the most are live), issued behind the first LDS
+  // reads and not where the compiler would, right before the use
+  u32x4 vf[4];
+  load_v(vf, cx, chunk_src(cx, ci), lane);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     const int set = b & 1;
@@ -1310,6 +1310,18 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
     for (int r = 0; r < 16; ++r) x[R][r] = v[r] - xg[r] * x[R][r];
     xh[2 * R] = split8<0>(x[R], xl[2 * R]);
     xh[2 * R + 1] = split8<1>(x[R], xl[2 * R + 1]);
+  }
+
+  // The state's decay of the second half, beside Delta's chains of products
+  // (which leave the vector unit idle), where no output accumulators take the
+  // registers (first segment launch of 1 x 16384 tokens at 4/8 heads 59.5 ->
+  // 54.6 us; with outputs it spills).
+  const float gl = Sc->row[kRowGl];
+  if constexpr (!OUT) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) st[t][r] *= gl;
   }
 
   // Delta = T diag(beta) X (T lower triangular: token blocks kb < 2 R + 2)
@@ -1351,7 +1363,6 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
   // Eight groups of products, each two key tiles' of one token block and one
   // of O's six lower blocks (three independent chains), their operands read a
   // group ahead.
-  const float gl = Sc->row[kRowGl];
   float qs[2], rq[2];
   if constexpr (OUT) {
 #pragma unroll
@@ -1395,7 +1406,7 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
   for (int i = 0; i < 8; ++i) {
     const int set = i & 1, t = 2 * (i >> 2), kb = i & 3;
     if (i < 7) read_group(i + 1, set ^ 1);
-    if (kb == 0) {
+    if (OUT && kb == 0) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -1690,6 +1701,11 @@ __device__ __forceinline__ void scan_body(Params p) {
 #pragma unroll
     for (int part = 0; part < 4; ++part)
       issue_part<OUT>(&In0, &S0, cx, first_src, part, wave - kScanWaves, lane);
+    // With the L2-norm the helpers' first half is the longer one: their
+    // instructions first (12 ragged sequences at 16/32 heads with it 173.5 ->
+    // 165.0 us a call; without the norm the main waves' chain is, 1-2% slower
+    // so).
+    if constexpr (L2) __builtin_amdgcn_s_setprio(2);
     wait_vmem();
     barrier_lds_no_dma();
     for (int ci = 0; ci < nchunks; ci += 2) {
