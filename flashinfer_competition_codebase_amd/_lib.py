@@ -156,9 +156,8 @@ def bind_host() -> None:
 
     with _lock:
         module.bind_decode(address(decode.gdn_decode_steps))
-        module.bind_prefill(address(prefill.gdn_prefill), address(prefill.gdn_prefill_noalloc),
-                            address(prefill.gdn_prefill_workspace_bytes),
-                            address(prefill.gdn_prefill_dispatches))
+        module.bind_prefill(address(prefill.gdn_prefill),
+                            address(prefill.gdn_prefill_workspace_bytes))
         bound_host = module
 
 

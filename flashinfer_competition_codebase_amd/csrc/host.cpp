@@ -5,7 +5,7 @@
 // us, and the Python checks of its twelve tensors, the workspace, the stream
 // and the 22-argument ctypes call made it 20.3 us a call; a value-returning
 // decode step of a few heads took 16.1.  These functions make the same checks,
-// allocations and call: 4.9 and 6.2 us.  They are a fast path only: arguments
+// allocations and call: 5.5 and 6.2 us.  They are a fast path only: arguments
 // outside what they accept (anything the Python path would refuse, convert or
 // treat specially) return None, nothing done, and the Python path takes the
 // call from the start, so its errors and conversions stay as they are.
@@ -34,9 +34,7 @@ constexpr int64_t kDim = 128;
 
 // The library functions, bound by bind_prefill and bind_decode.
 decltype(&gdn_prefill) g_prefill;
-decltype(&gdn_prefill_noalloc) g_prefill_noalloc;
 decltype(&gdn_prefill_workspace_bytes) g_workspace;
-decltype(&gdn_prefill_dispatches) g_dispatches;
 decltype(&gdn_decode_steps) g_decode;
 
 // A plain strided tensor in device memory: no subclass, and none of the
@@ -158,33 +156,20 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     output = &out_t;
     new_state = &state_t;
   }
-  // One launch (the token-by-token or the one-chunk kernel) reads no
-  // workspace: the entry that takes none.  Else the workspace is the current
-  // stream's, as the launch is: freed here, its memory is reused in that
-  // stream's order.
-  const bool no_workspace =
-      g_dispatches(l, n, hv) == 1 && need <= GDN_PREFILL_NOALLOC_SCRATCH_BYTES;
-  void* ws = nullptr;
-  if (!no_workspace) {
-    workspace = at::empty({static_cast<int64_t>(need + 256)},
-                          q->options().dtype(at::kByte).requires_grad(false));
-    ws = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(workspace.data_ptr()) + 255) &
-                                 ~static_cast<uintptr_t>(255));
-  }
+  // The workspace is the current stream's, as the launch is: freed here, its
+  // memory is reused in that stream's order.
+  workspace = at::empty({static_cast<int64_t>(need + 256)},
+                        q->options().dtype(at::kByte).requires_grad(false));
+  void* const ws = reinterpret_cast<void*>(
+      (reinterpret_cast<uintptr_t>(workspace.data_ptr()) + 255) & ~static_cast<uintptr_t>(255));
   void* const hip_stream = c10::hip::getCurrentHIPStream(q->device().index()).stream();
   const int l2 = args[12] == Py_True;
   int code;
   Py_BEGIN_ALLOW_THREADS;
-  if (no_workspace)
-    code = g_prefill_noalloc(ptr<void>(q), ptr<void>(k), ptr<void>(v), ptr<float>(state),
-                             ptr<float>(A_log), ptr<void>(a), ptr<float>(dt_bias), ptr<void>(b),
-                             ptr<int32_t>(cu), scale, ptr<void>(output), ptr<float>(new_state), l,
-                             n, h, hv, kDim, kDim, l2, hip_stream);
-  else
-    code = g_prefill(ptr<void>(q), ptr<void>(k), ptr<void>(v), ptr<float>(state),
-                     ptr<float>(A_log), ptr<void>(a), ptr<float>(dt_bias), ptr<void>(b),
-                     ptr<int32_t>(cu), scale, ptr<void>(output), ptr<float>(new_state), l, n, h,
-                     hv, kDim, kDim, l2, ws, need, hip_stream);
+  code = g_prefill(ptr<void>(q), ptr<void>(k), ptr<void>(v), ptr<float>(state),
+                   ptr<float>(A_log), ptr<void>(a), ptr<float>(dt_bias), ptr<void>(b),
+                   ptr<int32_t>(cu), scale, ptr<void>(output), ptr<float>(new_state), l, n, h, hv,
+                   kDim, kDim, l2, ws, need, hip_stream);
   Py_END_ALLOW_THREADS;
   // as the Python path: cu_seqlens may be another stream's tensor
   cu->record_stream(stream);
@@ -253,15 +238,13 @@ PyObject* decode_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind_prefill(gdn_prefill, gdn_prefill_noalloc, gdn_prefill_workspace_bytes,
-// gdn_prefill_dispatches) and bind_decode(gdn_decode_steps): addresses.
+// bind_prefill(gdn_prefill, gdn_prefill_workspace_bytes) and
+// bind_decode(gdn_decode_steps): addresses.
 PyObject* bind_prefill(PyObject*, PyObject* args) {
-  unsigned long long p, n, w, d;
-  if (!PyArg_ParseTuple(args, "KKKK", &p, &n, &w, &d)) return nullptr;
+  unsigned long long p, w;
+  if (!PyArg_ParseTuple(args, "KK", &p, &w)) return nullptr;
   g_prefill = reinterpret_cast<decltype(g_prefill)>(static_cast<uintptr_t>(p));
-  g_prefill_noalloc = reinterpret_cast<decltype(g_prefill_noalloc)>(static_cast<uintptr_t>(n));
   g_workspace = reinterpret_cast<decltype(g_workspace)>(static_cast<uintptr_t>(w));
-  g_dispatches = reinterpret_cast<decltype(g_dispatches)>(static_cast<uintptr_t>(d));
   Py_RETURN_NONE;
 }
 

@@ -46,7 +46,7 @@ PREFILLS = {
     "two launches": ([65, 7], 4, 8, True),
     "offsets kernel": ([70] + [1] * 70, 4, 8, False),
     "segments": ([1024], 2, 4, True),
-    "scratch too small for a token-path workspace": ([56], 256, 256, True),
+    "token path, many heads": ([56], 256, 256, True),
 }
 
 
@@ -136,3 +136,27 @@ def test_calls_the_native_path_leaves_to_python(hip_device):
         assert _lib.bound_host.decode_run(*args, False) is None, n
         with pytest.raises((TypeError, ValueError)):
             gdn.run(*args)
+
+
+@pytest.mark.parametrize("lens", [[6], [64], [65, 7]])
+def test_captured_prefill_replays(lens, hip_device):
+    """A prefill captured by torch after one eager call (which binds the
+    native path): replays over new inputs equal the eager results."""
+    _announce(f"captured prefill lens={lens}")
+    H, HV = 4, 8
+    t = _dev(make_prefill_inputs(lens, H, HV, seed=831), hip_device)
+    out, st = torch.empty_like(t["v"]), torch.empty_like(t["state"])
+    gdn.kernel_prefill_hip(**t, output=out, new_state=st)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gdn.kernel_prefill_hip(**t, output=out, new_state=st)
+    for rnd in range(3):
+        fresh = _dev(make_prefill_inputs(lens, H, HV, seed=840 + rnd), hip_device)
+        for n in ("q", "k", "v", "state", "a", "b"):
+            t[n].copy_(fresh[n])
+        graph.replay()
+        torch.cuda.synchronize()
+        ref_o, ref_s = gdn.prefill_run(**t)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref_o) and torch.equal(st, ref_s), rnd
