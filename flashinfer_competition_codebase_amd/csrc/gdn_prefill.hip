@@ -211,20 +211,17 @@ __device__ __forceinline__ void split4(const f32x4& x, s16x4& hi, s16x4& lo) {
   lo = __builtin_bit_cast(s16x4, l);
 }
 
-// Workgroup barrier that orders LDS only.  The waves of these kernels
-// exchange data through LDS alone, so global loads issued ahead of a barrier
-// (the next chunk's operands) stay in flight across it instead of being
-// drained as __syncthreads' all-memory fence would.
 // The wavefront's index in its workgroup, as a value the compiler knows is
 // the same in every lane (a scalar register): branches on it are scalar
-// branches and LDS bases derived from it need no per-lane waterfall.  Used by
-// the scan (64 x 512 qk16_v32: scan 485.9 -> 457.8 us with the L2-norm as a
-// template flag); the preparation kernel keeps threadIdx.x >> 6, with which
-// it measured faster (118.8 against 138.9 us).
+// branches and LDS bases derived from it need no per-lane waterfall.
 __device__ __forceinline__ int wave_index() {
   return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
 }
 
+// Workgroup barrier that orders LDS only.  The waves of these kernels
+// exchange data through LDS alone, so global loads issued ahead of a barrier
+// stay in flight across it instead of being drained as __syncthreads'
+// all-memory fence would.
 __device__ __forceinline__ void block_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
@@ -536,7 +533,7 @@ __device__ __forceinline__ float decay(float xh, float xl, float yh, float yl) {
 // trips, 12 KiB of K rows and two 64 x 64 matrices there limited a CU to four
 // such chains, and each diagonal block's substitution used 16 of 64 lanes.  A
 // wave of its own needs no barrier, keeps K K^T's operands and every block in
-// registers in the two layouts the products read (6 KiB of LDS and 149
+// registers in the two layouts the products read (6 KiB of LDS and 155
 // registers: twelve chains a CU), and runs the four substitutions at once.  Kernel
 // trace, before and after: 64 x 512 tokens at 16/32 heads 112-119 -> 82 us (4.5
 // TB/s of K rows in and slots out), 12 ragged sequences there 43 -> 28 us, 16 x
