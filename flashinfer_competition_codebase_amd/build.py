@@ -53,6 +53,7 @@ DECODE_SOURCES = ("flashinfer_competition_codebase_amd/csrc/gdn_decode_kernel.h"
                   "flashinfer_competition_codebase_amd/csrc/gdn_decode.hip",
                   "flashinfer_competition_codebase_amd/build.py")
 PREFILL_SOURCES = ("flashinfer_competition_codebase_amd/csrc/gdn_prefill.hip",
+                   "flashinfer_competition_codebase_amd/csrc/gdn_prefill_segments.h",
                    "flashinfer_competition_codebase_amd/csrc/gdn_decode_kernel.h",
                    "flashinfer_competition_codebase_amd/build.py")
 

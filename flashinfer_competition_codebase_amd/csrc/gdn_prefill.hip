@@ -86,6 +86,7 @@
 
 #include "gdn_decode_kernel.h"
 #include "gdn_prefill.h"
+#include "gdn_prefill_segments.h"
 
 namespace gdn_pf {
 
@@ -278,7 +279,8 @@ struct Params {
   // blocks in k-last order (element (k, c) at c * 128 + k).
   int seg_chunks;            // chunks per segment, 0: no segments
   int nseg;                  // segments
-  float* seg_S;              // [nseg, HV] state at each segment's start (1 .. nseg-1)
+  float* seg_S;              // [nseg, HV] state at each segment's start (1 .. nseg-1;
+                             // in place 0 too)
   float* seg_B;              // [nseg, HV] state at its end from a zero start
   float* seg_M;              // [nseg, HV] its transition: end = M start + B (M[k][k'])
   // > 0: the token-by-token kernel was launched first with this limit (at
@@ -1497,8 +1499,9 @@ __device__ __forceinline__ void store_end(float* st_out, bool transition, const 
 // segment 0 from the sequence's state (end: seg_S[1]) and segments
 // 1 .. nseg-2 from a zero start (end: seg_B) and from the identity without
 // values (end: seg_M, as the combine's operand); the second (OUT) runs every
-// segment from its start (segment 0: the sequence's state, then seg_S) with
-// the outputs, the last one's end being the new state.
+// segment from its start (segment 0: the sequence's state -- in place, seg_S[0],
+// the first launch's copy of it -- then seg_S) with the outputs, the last one's
+// end being the new state (seg_unit).
 template <bool FEW, bool SEG, bool OUT, bool L2, bool FUSE>
 __device__ __forceinline__ void scan_body(Params p) {
   static_assert(OUT || SEG, "only segments run without outputs");
@@ -1535,6 +1538,7 @@ __device__ __forceinline__ void scan_body(Params p) {
   const float* st_in = nullptr;       // null: zeros (or the identity)
   bool identity = false, values = true, pass_through = false;
   float* st_out;
+  float* st_keep = nullptr;           // where the start is copied to
   int s = 0, start, end, slot0 = 0, nchunks = 0;
   // the sequence's chunk slots (never more than its range holds, and never
   // more slots than the workspace has, whatever cu_seqlens contains)
@@ -1566,27 +1570,23 @@ __device__ __forceinline__ void scan_body(Params p) {
     auto seg_blk = [&](float* base, int sg) {
       return base + (static_cast<size_t>(sg) * p.HV + hv) * blk;
     };
-    int j;
-    if (!OUT) {
-      const int mid = nseg - 2;                   // segments 1 .. nseg-2
-      if (u == 0) {
-        j = 0;
-        st_in = p.state ? p.state + sh * blk : nullptr;
-        st_out = seg_blk(p.seg_S, g0 + 1);
-      } else if (u <= mid) {
-        j = u;
-        st_out = seg_blk(p.seg_B, g0 + j);
-      } else {
-        j = u - mid;
-        identity = true;
-        values = false;
-        st_out = seg_blk(p.seg_M, g0 + j);
-      }
-    } else {
-      j = u;
-      st_in = j == 0 ? (p.state ? p.state + sh * blk : nullptr) : seg_blk(p.seg_S, g0 + j);
-      st_out = j == nseg - 1 ? p.new_state + sh * blk : nullptr;
+    const SegUnit un = seg_unit(OUT, nseg, u, p.state != nullptr && p.state == p.new_state);
+    const int j = un.seg;
+    if (un.from == SegBlock::kState)
+      st_in = p.state ? p.state + sh * blk : nullptr;
+    else if (un.from == SegBlock::kStart)
+      st_in = seg_blk(p.seg_S, g0 + j);
+    if constexpr (OUT) {
+      st_out = un.to == SegBlock::kNewState ? p.new_state + sh * blk : nullptr;
       pass_through = j > 0;
+    } else {
+      identity = un.from == SegBlock::kIdentity;
+      values = !identity;
+      st_out = seg_blk(un.to == SegBlock::kStart     ? p.seg_S
+                       : un.to == SegBlock::kZeroEnd ? p.seg_B
+                                                     : p.seg_M,
+                       g0 + un.to_seg);
+      if (un.keep_start) st_keep = seg_blk(p.seg_S, g0 + j);
     }
     int base, count;
     seq_slots(s, base, count);
@@ -1635,6 +1635,10 @@ __device__ __forceinline__ void scan_body(Params p) {
   for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
     for (int e = 0; e < 8; ++e) sel[h2][e] = perm32(m) == 16 * h2 + 8 * g + e ? 0x3f80 : 0;
+
+  if constexpr (SEG && !OUT) {
+    if (st_keep != nullptr && wave < kScanWaves) store_end(st_keep, false, st, sel);
+  }
 
   // No tokens: a sequence ends in zeros, as the reference; a segment with no
   // chunk slots (a malformed batch whose slots ran past the workspace's)
@@ -2047,8 +2051,11 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
       !aligned(a, 2) || !aligned(b, 2))
     return hipErrorInvalidValue;
   if (state != nullptr && state == new_state) {
-    // in place is fine: each scan workgroup reads its state slice before
-    // writing it, and no two workgroups share a slice
+    // in place is fine: a workgroup of the token path and of the plain scan
+    // reads its state slice before writing it, and no two workgroups share a
+    // slice; in segments, whose first and last are scanned by different
+    // workgroups of one launch, the first starts from a copy that the launch
+    // before made
   } else if (state != nullptr) {
     const uintptr_t s0 = reinterpret_cast<uintptr_t>(state);
     const uintptr_t d0 = reinterpret_cast<uintptr_t>(new_state);

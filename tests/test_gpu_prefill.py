@@ -209,6 +209,27 @@ def test_segmented_in_place_and_timed(hip_device):
             hip.hipEventDestroy(e)
 
 
+@pytest.mark.parametrize("lens,H,HV,l2", [
+    ([384], 4, 8, False),                    # the fewest segments
+    ([900, 20, 1300], 2, 2, True),           # a one-segment sequence among them
+    ([1500, 0, 700, 3000], 4, 8, False),     # an empty sequence
+    ([5000, 4100, 6000, 3900, 5200, 4800, 5500, 4903], 4, 8, False),   # offsets kernel
+])
+def test_segmented_sequences_in_place(lens, H, HV, l2, hip_device):
+    """In place, segment 0 starts from the copy of its state that the first
+    launch keeps: the same bits as out of place, call after call."""
+    _announce(f"segmented prefill in place lens={lens} H={H} HV={HV} l2={l2}")
+    assert gdn.prefill.prefill_dispatches(sum(lens), len(lens), HV) >= 4
+    t = _dev(make_prefill_inputs(lens, H, HV, seed=420 + sum(lens), unit_qk=not l2), hip_device)
+    state, out = t["state"].clone(), torch.empty_like(t["v"])
+    for _ in range(2):
+        ref_o, ref_s = gdn.prefill_run(**{**t, "state": state}, use_qk_l2norm=l2)
+        gdn.kernel_prefill_hip(**{**t, "state": state}, output=out, new_state=state,
+                               use_qk_l2norm=l2)
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref_o) and torch.equal(state, ref_s)
+
+
 def test_l2norm_and_no_state(hip_device):
     _announce("prefill l2norm, state=None, raw-scale q/k")
     t = make_prefill_inputs([40, 90], 4, 8, seed=12, with_state=False, unit_qk=False)
