@@ -229,6 +229,16 @@ __device__ __forceinline__ void block_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The same among the lanes of one wave, whose LDS accesses are carried out in
+// program order: no instruction, but the fences keep the compiler from moving
+// an access across (the barrier alone is no memory operation, and what one
+// lane stores and another loads looks unrelated in each lane's own view).
+__device__ __forceinline__ void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
@@ -653,11 +663,11 @@ __device__ __forceinline__ void prep_chunk(const Params& p, int c, int t0, int n
     const double gamma64 = wave_prefix_sum(static_cast<double>(log2g));
     const float gamma = static_cast<float>(gamma64);
     const float gamma_lo = static_cast<float>(gamma64 - static_cast<double>(gamma));
-    __builtin_amdgcn_wave_barrier();
+    wave_sync_lds();
     lds.gamma[lane] = gamma;
     lds.gamma_lo[lane] = gamma_lo;
     lds.beta[lane] = beta;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync_lds();
 
     // A's blocks below the diagonal, row layout; the diagonal ones (strictly
     // lower) by rows to LDS.  The decays are computed for every element with
@@ -687,7 +697,7 @@ __device__ __forceinline__ void prep_chunk(const Params& p, int c, int t0, int n
       }
       *reinterpret_cast<f32x4*>(&lds.blk[r][i * kBlkStride + 4 * g]) = A[r * (r + 1) / 2 + r];
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync_lds();
 
     // T = (I + A)^-1 by block recursion on 16 x 16 blocks (A is strictly lower
     // triangular, so T is unit lower triangular):
@@ -715,12 +725,12 @@ __device__ __forceinline__ void prep_chunk(const Params& p, int c, int t0, int n
         }
         t[r] = s0 + s1;
       }
-      __builtin_amdgcn_wave_barrier();
+      wave_sync_lds();
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f32x4*>(&lds.blk[g][i * kBlkStride + 4 * q]) =
             f32x4{t[4 * q], t[4 * q + 1], t[4 * q + 2], t[4 * q + 3]};
-      __builtin_amdgcn_wave_barrier();
+      wave_sync_lds();
     }
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
@@ -1138,8 +1148,7 @@ __device__ __forceinline__ void p_tile_store(const f32x4& acc, const ScanScales*
 template <bool OUT, bool L2>
 __device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
                                            const ScanScales* __restrict__ Sc,
-                                           uint16_t* __restrict__ Kt, uint16_t* __restrict__ Pb,
-                                           float* __restrict__ Qn,
+                                           uint16_t* Kt, uint16_t* Pb, float* Qn,
                                            const uint16_t* __restrict__ Sel, int w, int lane) {
   const int m = lane & 31, g = lane >> 5;
   const unsigned row0 = static_cast<unsigned>(m) * kDim + 8u * (g ^ (m & 15));
@@ -1195,15 +1204,17 @@ __device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
 
 // Chunk ci of a helper wave: the side tiles from In and Sc, then the next
 // chunk's DMA into InN and ScN (their last reads were in the chunk before).
-// All pointers are restrict: the compiler then knows that the DMA never
-// writes what is read meanwhile, and waits for it only at the end.
+// The pointers to the chunks' inputs are restrict: the compiler then knows
+// that the DMA never writes what is read meanwhile, and waits for it only at
+// the end.  Kt, Pb and Qn are not: the other waves access them within the
+// call, on the other side of its barriers.
 template <bool OUT, bool L2>
 __device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
                                            const ScanScales* __restrict__ Sc,
                                            ScanIn<OUT>* __restrict__ InN,
                                            ScanScales* __restrict__ ScN,
-                                           uint16_t* __restrict__ Kt, uint16_t* __restrict__ Pb,
-                                           float* __restrict__ Qn, const ScanCtx& cx,
+                                           uint16_t* Kt, uint16_t* Pb, float* Qn,
+                                           const ScanCtx& cx,
                                            const uint16_t* __restrict__ Sel, int ci) {
   const int lane = threadIdx.x & 63;
   const int w = wave_index() - kScanWaves;
@@ -1223,7 +1234,8 @@ __device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
 
 // Chunk ci of a main wave, from In and Sc (LAST: the last chunk, which may be
 // a partial one); Kt: the K^T operand blocks; Pb: the P' operand blocks
-// (OUT); Qn: the Q row scales (L2).  OUT: the outputs too (else only the
+// (OUT); Qn: the Q row scales (L2) -- written by the helper waves before the
+// call's first barrier, so not restrict.  OUT: the outputs too (else only the
 // state).  L2: the L2-norm.
 //
 // The output's intra-chunk term uses P = diag(rq) P' with
@@ -1236,9 +1248,8 @@ __device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
 template <bool OUT, bool L2, bool LAST>
 __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
                                            const ScanScales* __restrict__ Sc,
-                                           const uint16_t* __restrict__ Kt,
-                                           const uint16_t* __restrict__ Pb,
-                                           const float* __restrict__ Qn, const ScanCtx& cx,
+                                           const uint16_t* Kt, const uint16_t* Pb,
+                                           const float* Qn, const ScanCtx& cx,
                                            f32x16 (&st)[4], const uint16_t* __restrict__ Sel,
                                            int ci) {
   // The lane index, opaque to the compiler: it would keep every LDS and

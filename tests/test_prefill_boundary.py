@@ -14,6 +14,7 @@ import torch
 import flashinfer_competition_codebase_amd as gdn
 from tests.gdn_cases import prefill_segment_plan
 from flashinfer_competition_codebase_amd import _lib
+from flashinfer_competition_codebase_amd.build import PREFILL_SRC
 from flashinfer_competition_codebase_amd.prefill import check_prefill_inputs
 from oracle.gdn_prefill_oracle import make_prefill_inputs
 
@@ -145,3 +146,18 @@ def test_entry_points_are_registered_like_the_reference():
     assert "prefill-hip-run" in gdn.NO_DPS and "prefill-hip" not in gdn.NO_DPS
     with pytest.raises(ValueError):
         gdn.prefill_run(**_cpu_inputs())      # CPU tensors: no CPU path
+
+
+def test_lds_exchanges_are_ordered_for_the_compiler():
+    """Lanes of a wave, and the scan's two kinds of waves, hand values to each
+    other through LDS.  A wave barrier is no memory operation, so each one
+    stands between a release and an acquire fence; and what other waves write
+    within a call is not handed to it as restrict."""
+    text = re.sub(r"//[^\n]*", "", PREFILL_SRC.read_text())
+    fenced = re.findall(r'__builtin_amdgcn_fence\(__ATOMIC_RELEASE, "wavefront", "local"\);\s*'
+                        r"__builtin_amdgcn_wave_barrier\(\);\s*"
+                        r'__builtin_amdgcn_fence\(__ATOMIC_ACQUIRE, "wavefront", "local"\);', text)
+    assert text.count("__builtin_amdgcn_wave_barrier") == len(fenced) > 0
+    for name in ("Kt", "Pb", "Qn"):
+        assert re.search(rf"\*\s*{name}\b", text), name
+        assert not re.search(rf"__restrict__\s+{name}\b", text), name
