@@ -489,12 +489,17 @@ __global__ __launch_bounds__(kThreads) void chunk_offsets_kernel(Params p, int32
 
 // Gates of token t, v-head hv: the decay's log2 and beta
 // (g = exp(-exp(A_log) softplus(a + dt_bias)), beta = sigmoid(b)).  The decays
-// stay in log2 units: each later exponential is one v_exp_f32.
+// stay in log2 units: each later exponential is one v_exp_f32.  A decay below
+// 2^kForgetLog2 is zero with or without the tokens beside it, so the log2 stops
+// there: the cumulative sums stay finite (a difference of two -inf is NaN) and
+// keep the other tokens' decays however large this one's is.  NaN passes.
+constexpr float kForgetLog2 = -1024.0f;
 __device__ __forceinline__ void gates_of(uint16_t a_raw, uint16_t b_raw, float dt_bias,
                                          float A_log, float& log2g, float& beta) {
   const float x = bf16_to_f32(a_raw) + dt_bias;
   const float sp = x > kSoftplusThreshold ? x * kLog2e : __builtin_amdgcn_logf(1.0f + __expf(x));
   log2g = -__expf(A_log) * sp;
+  log2g = log2g < kForgetLog2 ? kForgetLog2 : log2g;
   beta = __builtin_amdgcn_rcpf(1.0f + __expf(-bf16_to_f32(b_raw)));
 }
 

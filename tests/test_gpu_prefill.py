@@ -758,3 +758,35 @@ def test_fast_forgetting_heads_keep_the_split_precision(lens, l2, hip_device):
     _, s64 = prefill_chunked_fp64(**t, use_qk_l2norm=l2)
     err = np.linalg.norm(st.cpu().double().numpy() - s64) / np.linalg.norm(s64)
     assert err < 2.0 ** -16, err
+
+
+@pytest.mark.parametrize("lens,H,HV,l2", [
+    ([57], 4, 8, False),                # the one-chunk kernel
+    ([64], 2, 6, True),
+    ([65, 7], 4, 8, False),             # chunk slots found in the kernels
+    ([70] + [1] * 70, 4, 8, True),      # the offsets kernel
+    ([384], 4, 8, False),               # segments
+    ([130, 1000], 2, 4, True),
+])
+@pytest.mark.parametrize("forget", ["inf", "max", "1e30", "A_log"])
+def test_tokens_that_forget_everything(lens, H, HV, l2, forget, hip_device):
+    """Tokens whose log-decay is -inf, or so large that a sum with it keeps
+    nothing of the others, forget the state exactly, as the recurrence does:
+    outputs and states equal those for the same inputs with a log-decay of
+    -2000 or below there (e^-2000 is zero in 64 bits too)."""
+    _announce(f"tokens that forget lens={lens[:4]} H={H} HV={HV} l2={l2} by {forget}")
+    t = make_prefill_inputs(lens, H, HV, seed=540 + sum(lens) + HV, unit_qk=not l2)
+    ref = dict(t)
+    if forget == "A_log":               # a head of which every token forgets
+        t["A_log"], ref["A_log"] = t["A_log"].clone(), t["A_log"].clone()
+        t["A_log"][HV - 1], ref["A_log"][HV - 1] = 100.0, 20.0
+    else:
+        value = {"inf": float("inf"), "max": torch.finfo(torch.bfloat16).max, "1e30": 1e30}[forget]
+        t["a"], ref["a"] = t["a"].clone(), t["a"].clone()
+        L = sum(lens)
+        for hv, tokens in ((0, (0,)), (1, (20, 21, 40)), (2, (31,)), (3, (63, 64)), (HV - 1, (L - 1,))):
+            for tok in tokens:
+                t["a"][min(tok, L - 1), hv], ref["a"][min(tok, L - 1), hv] = value, 4000.0
+    out, st = gdn.prefill_run(**_dev(t, hip_device), use_qk_l2norm=l2)
+    torch.cuda.synchronize()
+    _check(ref, out, st, l2=l2)
