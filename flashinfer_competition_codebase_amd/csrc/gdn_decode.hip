@@ -47,7 +47,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <iterator>
 #include <new>
+#include <utility>
 
 #include "gdn_decode.h"
 #include "gdn_decode_block.h"
@@ -490,17 +492,31 @@ int group_layers(const StepArgs* const* args, int n) {
   return count;
 }
 
-template <int NS, int W, bool BF16>
-hipError_t launch_layers_one(const StepArgs& s, int count, const LayerTable& t, hipStream_t stream) {
-  const unsigned ratio = static_cast<unsigned>(s.HV / s.H);
-  const unsigned z = static_cast<unsigned>(count) * static_cast<unsigned>(s.B);
-  const dim3 grid(ratio * (kDim / (kLaneGroups * NS * W)), static_cast<unsigned>(s.H), z);
-  auto* kern = s.use_qk_l2norm != 0 ? gdn_decode_layers_k128<NS, W, true, BF16>
-                                    : gdn_decode_layers_k128<NS, W, false, BF16>;
-  const unsigned h_ratio = static_cast<unsigned>(s.H) | (ratio << 16) |
-                           (z >= kGroupMinSeqs ? kGroupFlag : 0u);
-  hipLaunchKernelGGL(kern, grid, dim3(64 * W), 0, stream, h_ratio, s.B, s.scale, t);
-  return hipGetLastError();
+// The layers kernel of a launch shape: one instance per row of the single-token
+// tables, taken from the tables themselves (null for any other shape).
+using LayersKernel = void (*)(unsigned, int, float, LayerTable);
+
+template <bool BF16>
+constexpr auto& layers_table() {
+  if constexpr (BF16) return kShapeBf16; else return kShapeFp32;
+}
+
+template <bool BF16, size_t... I>
+LayersKernel layers_kernel(int ns, int w, bool l2, std::index_sequence<I...>) {
+  constexpr auto& table = layers_table<BF16>();
+  LayersKernel kern = nullptr;
+  ((table[I].ns == ns && table[I].waves == w
+        ? void(kern = l2 ? gdn_decode_layers_k128<table[I].ns, table[I].waves, true, BF16>
+                         : gdn_decode_layers_k128<table[I].ns, table[I].waves, false, BF16>)
+        : void()),
+   ...);
+  return kern;
+}
+
+template <bool BF16>
+LayersKernel layers_kernel(int ns, int w, bool l2) {
+  return layers_kernel<BF16>(ns, w, l2,
+                             std::make_index_sequence<std::size(layers_table<BF16>())>());
 }
 
 // The layers' launch, with the single-token launch shape of all their heads
@@ -517,25 +533,18 @@ hipError_t launch_layers(const StepArgs* const* args, int count, hipStream_t str
   }
   int ns = 0, w = 0, policy = 0;
   choose_shape(static_cast<long long>(count) * s.B * s.HV, s.state_bf16 != 0, 1, &ns, &w, &policy);
-  if (s.state_bf16 == 0) {
-    switch (ns * 16 + w) {                         // the rows of kShapeFp32
-      case 1 * 16 + 1: return launch_layers_one<1, 1, false>(s, count, t, stream);
-      case 2 * 16 + 2: return launch_layers_one<2, 2, false>(s, count, t, stream);
-      case 4 * 16 + 1: return launch_layers_one<4, 1, false>(s, count, t, stream);
-      case 8 * 16 + 1: return launch_layers_one<8, 1, false>(s, count, t, stream);
-      case 2 * 16 + 4: return launch_layers_one<2, 4, false>(s, count, t, stream);
-      default: return hipErrorInvalidValue;
-    }
-  }
-  switch (ns * 16 + w) {                           // the rows of kShapeBf16
-    case 1 * 16 + 2: return launch_layers_one<1, 2, true>(s, count, t, stream);
-    case 1 * 16 + 4: return launch_layers_one<1, 4, true>(s, count, t, stream);
-    case 2 * 16 + 4: return launch_layers_one<2, 4, true>(s, count, t, stream);
-    case 2 * 16 + 2: return launch_layers_one<2, 2, true>(s, count, t, stream);
-    case 2 * 16 + 1: return launch_layers_one<2, 1, true>(s, count, t, stream);
-    case 4 * 16 + 4: return launch_layers_one<4, 4, true>(s, count, t, stream);
-    default: return hipErrorInvalidValue;
-  }
+  const bool l2 = s.use_qk_l2norm != 0;
+  const LayersKernel kern =
+      s.state_bf16 ? layers_kernel<true>(ns, w, l2) : layers_kernel<false>(ns, w, l2);
+  if (kern == nullptr) return hipErrorInvalidValue;   // not reached: the shape is a row
+  const unsigned ratio = static_cast<unsigned>(s.HV / s.H);
+  const unsigned z = static_cast<unsigned>(count) * static_cast<unsigned>(s.B);
+  const dim3 grid(ratio * static_cast<unsigned>(kDim / (kLaneGroups * ns * w)),
+                  static_cast<unsigned>(s.H), z);
+  const unsigned h_ratio = static_cast<unsigned>(s.H) | (ratio << 16) |
+                           (z >= kGroupMinSeqs ? kGroupFlag : 0u);
+  hipLaunchKernelGGL(kern, grid, dim3(64 * w), 0, stream, h_ratio, s.B, s.scale, t);
+  return hipGetLastError();
 }
 
 StepArgs make_args(const void* q, const void* k, const void* v, const void* state,

@@ -261,6 +261,35 @@ def test_graph_of_equal_layers_matches_eager_bits(n_layers, B, H, HV, dtype, l2,
     _same_bits_graph_and_eager(make, l2=l2)
 
 
+def _equal_layers(n_layers, B, H, HV, dtype, device, seed):
+    """Layers of one size, each its own buffers, every other one in place."""
+    dev = []
+    for i in range(n_layers):
+        t = make_inputs(B, H, HV, seed=seed + i)
+        d = {n: (x.to(device) if isinstance(x, torch.Tensor) else x) for n, x in t.items()}
+        d["state"] = d["state"].to(dtype)
+        d["new_state"] = d["state"] if i % 2 == 0 else torch.empty_like(d["state"])
+        d["output"] = torch.empty(B, 1, HV, 128, dtype=torch.bfloat16, device=device)
+        dev.append(d)
+    return dev
+
+
+@pytest.mark.parametrize("n_layers,B,H,HV,dtype", [
+    (2, 1, 4, 16, torch.bfloat16),             # 32 heads in all: 1 row x 4 waves
+    (4, 1, 4, 16, torch.bfloat16),             # 64: 2 x 4
+    (8, 1, 4, 16, torch.bfloat16),             # 128: 2 x 2
+    (16, 1, 4, 16, torch.bfloat16),            # 256: 2 x 1
+    (8, 1, 4, 8, torch.float32),               # 64: 2 x 2
+    (3, 45, 16, 32, torch.float32),            # past 4096 heads: 2 x 2, grouped by XCD
+    (3, 45, 16, 32, torch.bfloat16),
+])
+def test_graph_of_equal_layers_by_launch_shape(n_layers, B, H, HV, dtype, hip_device):
+    """The rows of the launch tables that the sizes above leave out."""
+    _announce(f"DecodeLayers launch shapes: {n_layers} x B={B} qk{H}_v{HV} {dtype}")
+    _same_bits_graph_and_eager(
+        lambda: _equal_layers(n_layers, B, H, HV, dtype, hip_device, 5600), n_steps=2)
+
+
 @pytest.mark.parametrize("link", ["output_to_v", "shared_state", "shared_output", "scale",
                                   "state_of_previous", "gates_in_state"])
 def test_graph_keeps_the_order_of_linked_layers(link, hip_device):
