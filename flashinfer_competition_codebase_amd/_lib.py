@@ -2,7 +2,7 @@
 in ``include/gdn_decode.h`` and ``include/gdn_prefill.h``).
 
 There is no fallback: if the library is missing or fails to load, every entry
-point raises ``RuntimeError`` naming the build command.  The reference builds
+point of it raises ``RuntimeError`` naming the build command.  The reference builds
 its native module lazily on first use (solution/cuda/binding.py:14-28); here
 the library is built ahead of time, in-tree, by ``build.py``.
 """
@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libgdn_decode.so"
@@ -135,30 +136,56 @@ def get_prefill_lib() -> ctypes.CDLL:
 
 
 # The native call path of the entry points (``_gdn_host``, csrc/host.cpp), once
-# bound to both libraries by the first call that passed the Python checks.
+# loaded by a call that passed the Python checks.  Each half is bound to its own
+# library and takes no calls before that.
 bound_host = None
+_host_error = None
+_host_halves: set = set()
 
 
-def bind_host() -> None:
-    """Load the native host module and bind it (once)."""
-    global bound_host
-    if bound_host is not None:
+def _load_host():
+    """The native host module.  It is compiled against one torch: a module that
+    does not import here, or was compiled against another version, is an
+    ImportError."""
+    import torch
+
+    from . import _gdn_host as module
+    if module.torch_version != torch.__version__:
+        raise ImportError(f"_gdn_host was compiled against torch {module.torch_version}, "
+                          f"not {torch.__version__}")
+    return module
+
+
+def bind_host(*, decode: bool = True, prefill: bool = True) -> None:
+    """Load the native host module and bind its decode and prefill halves (each
+    once).  It only shortens the call: where it does not load, one warning says
+    so and every call keeps the ctypes path to the same libraries."""
+    global bound_host, _host_error
+    if (_host_error is not None or
+            (decode <= ("decode" in _host_halves) and prefill <= ("prefill" in _host_halves))):
         return
-    decode, prefill = get_lib(), get_prefill_lib()
     try:
-        from . import _gdn_host as module
+        module = _load_host()
     except ImportError as exc:
-        raise RuntimeError(f"native host module not loadable ({exc}); build it with "
-                           "`python -m flashinfer_competition_codebase_amd.build`") from exc
+        _host_error = exc
+        warnings.warn(f"native host module not loadable ({exc}); calls take the slower Python "
+                      "path to the libraries.  Build it with "
+                      "`python -m flashinfer_competition_codebase_amd.build`", RuntimeWarning,
+                      stacklevel=2)
+        return
 
     def address(fn):
         return ctypes.cast(fn, ctypes.c_void_p).value
 
-    with _lock:
-        module.bind_decode(address(decode.gdn_decode_steps))
-        module.bind_prefill(address(prefill.gdn_prefill),
-                            address(prefill.gdn_prefill_workspace_bytes))
-        bound_host = module
+    if decode:
+        lib = get_lib()
+        module.bind_decode(address(lib.gdn_decode_steps))
+        _host_halves.add("decode")
+    if prefill:
+        lib = get_prefill_lib()
+        module.bind_prefill(address(lib.gdn_prefill), address(lib.gdn_prefill_workspace_bytes))
+        _host_halves.add("prefill")
+    bound_host = module
 
 
 _raw_stream = None

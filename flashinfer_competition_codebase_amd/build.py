@@ -113,6 +113,7 @@ def host_compile_command(out: Path = HOST_PATH, src: Path = HOST_SRC) -> list[st
     lib = Path(torch.__file__).resolve().parent / "lib"
     return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DGDN_TORCH_VERSION="{torch.__version__}"',
             *[f"-isystem{p}" for p in cpp_extension.include_paths()],
             f"-isystem{sysconfig.get_paths()['include']}", f"-isystem{rocm}/include",
             f"-I{INCLUDE_DIR}",

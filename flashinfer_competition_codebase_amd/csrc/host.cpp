@@ -268,4 +268,13 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_gdn_host", nullptr, -1, kMethods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__gdn_host(void) { return PyModule_Create(&kModule); }
+// torch_version: the torch that the module was compiled against (its inline
+// accessors know that one's object layouts), for the importer to compare.
+PyMODINIT_FUNC PyInit__gdn_host(void) {
+  PyObject* const m = PyModule_Create(&kModule);
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", GDN_TORCH_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -384,7 +384,7 @@ def _run_checked(q, k, v, state, A_log, a, dt_bias, b, scale, use_qk_l2norm):
     output = torch.empty((B, T, HV, V_DIM), dtype=torch.bfloat16, device=q.device)
     new_state = torch.empty((B, HV, V_DIM, K_DIM), dtype=sdtype, device=q.device)
     if B > 0:
-        _lib.bind_host()               # calls like this one run natively from here on
+        _lib.bind_host(prefill=False)  # calls like this one run natively from here on
         # fresh outputs every call: launched directly, not bound for reuse
         _launch(q, k, v, state, A_log, a, dt_bias, b, resolve_scale(scale, q.shape[-1]),
                 output, new_state, B, T, H, HV, use_qk_l2norm)

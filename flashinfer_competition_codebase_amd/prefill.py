@@ -200,7 +200,7 @@ def _launch(q, k, v, state, A_log, a, dt_bias, b, cu_seqlens, scale, output, new
         return None
     if cu_seqlens.dtype != torch.int32:
         cu_seqlens = cu_seqlens.to(torch.int32)
-    _lib.bind_host()                   # calls like this one run natively from here on
+    _lib.bind_host(decode=False)       # calls like this one run natively from here on
     lib = _lib.get_prefill_lib()
     ws_bytes = workspace_bytes(L, N, H, HV)
     workspace = torch.empty(ws_bytes + 256, dtype=torch.uint8, device=q.device)
