@@ -92,9 +92,17 @@ bool ranges_overlap(const at::Tensor* x, const at::Tensor* y) {
   return x0 < y0 + y->nbytes() && y0 < x0 + x->nbytes();
 }
 
+// A tensor the call reads.
 template <typename T>
-T* ptr(const at::Tensor* t) {
-  return t == nullptr ? nullptr : static_cast<T*>(const_cast<void*>(t->const_data_ptr()));
+const T* ptr(const at::Tensor* t) {
+  return t == nullptr ? nullptr : static_cast<const T*>(t->const_data_ptr());
+}
+
+// A tensor the call writes: one that shares its memory until it is written (a
+// lazy clone) gets its own first, on the current stream.
+template <typename T>
+T* out_ptr(const at::Tensor* t) {
+  return static_cast<T*>(t->mutable_data_ptr());
 }
 
 PyObject* code_of(int code) {
@@ -140,11 +148,14 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                     !is(new_state, at::kFloat, {N, HV, kDim, kDim})))
     Py_RETURN_NONE;
   if (!one_device(q, {k, v, state, A_log, a, dt_bias, b, cu, output, new_state})) Py_RETURN_NONE;
-  if (state != nullptr && new_state != nullptr &&
-      new_state->const_data_ptr() != state->const_data_ptr() && ranges_overlap(new_state, state))
-    Py_RETURN_NONE;
   c10::Stream stream(c10::Stream::DEFAULT, q->device());
   if (!stream_of(q, &stream)) Py_RETURN_NONE;
+  if (!allocate) {
+    out_ptr<void>(output);                         // before any pointer is compared
+    const void* const d = out_ptr<void>(new_state);
+    if (state != nullptr && d != state->const_data_ptr() && ranges_overlap(new_state, state))
+      Py_RETURN_NONE;
+  }
   const int n = static_cast<int>(N), l = static_cast<int>(L), h = static_cast<int>(H),
             hv = static_cast<int>(HV);
   const size_t need = g_workspace(l, n, h, hv);
@@ -164,12 +175,17 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       (reinterpret_cast<uintptr_t>(workspace.data_ptr()) + 255) & ~static_cast<uintptr_t>(255));
   void* const hip_stream = c10::hip::getCurrentHIPStream(q->device().index()).stream();
   const int l2 = args[12] == Py_True;
+  // the pointers before the interpreter lock is released: an accessor may throw
+  const void *qp = ptr<void>(q), *kp = ptr<void>(k), *vp = ptr<void>(v), *ap = ptr<void>(a),
+             *bp = ptr<void>(b);
+  const float *sp = ptr<float>(state), *lp = ptr<float>(A_log), *dp = ptr<float>(dt_bias);
+  const int32_t* const cp = ptr<int32_t>(cu);
+  void* const op = out_ptr<void>(output);
+  float* const np = out_ptr<float>(new_state);
   int code;
   Py_BEGIN_ALLOW_THREADS;
-  code = g_prefill(ptr<void>(q), ptr<void>(k), ptr<void>(v), ptr<float>(state),
-                   ptr<float>(A_log), ptr<void>(a), ptr<float>(dt_bias), ptr<void>(b),
-                   ptr<int32_t>(cu), scale, ptr<void>(output), ptr<float>(new_state), l, n, h, hv,
-                   kDim, kDim, l2, ws, need, hip_stream);
+  code = g_prefill(qp, kp, vp, sp, lp, ap, dp, bp, cp, scale, op, np, l, n, h, hv, kDim, kDim, l2,
+                   ws, need, hip_stream);
   Py_END_ALLOW_THREADS;
   // as the Python path: cu_seqlens may be another stream's tensor
   cu->record_stream(stream);
@@ -222,12 +238,15 @@ PyObject* decode_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       at::empty({B, HV, kDim, kDim}, (bf16 ? q : A_log)->options().requires_grad(false));
   void* const hip_stream = c10::hip::getCurrentHIPStream(q->device().index()).stream();
   const int l2 = args[9] == Py_True;
+  const void *qp = ptr<void>(q), *kp = ptr<void>(k), *vp = ptr<void>(v), *sp = ptr<void>(state),
+             *ap = ptr<void>(a), *bp = ptr<void>(b);
+  const float *lp = ptr<float>(A_log), *dp = ptr<float>(dt_bias);
+  void *const op = out_ptr<void>(&output), *const np = out_ptr<void>(&new_state);
   int code;
   Py_BEGIN_ALLOW_THREADS;
-  code = g_decode(ptr<void>(q), ptr<void>(k), ptr<void>(v), ptr<void>(state), ptr<float>(A_log),
-                  ptr<void>(a), ptr<float>(dt_bias), ptr<void>(b), scale, ptr<void>(&output),
-                  ptr<void>(&new_state), static_cast<int>(B), static_cast<int>(T),
-                  static_cast<int>(H), static_cast<int>(HV), kDim, kDim, bf16, l2, hip_stream);
+  code = g_decode(qp, kp, vp, sp, lp, ap, dp, bp, scale, op, np, static_cast<int>(B),
+                  static_cast<int>(T), static_cast<int>(H), static_cast<int>(HV), kDim, kDim, bf16,
+                  l2, hip_stream);
   Py_END_ALLOW_THREADS;
   PyObject* const r = PyTuple_New(3);
   if (r == nullptr) return nullptr;

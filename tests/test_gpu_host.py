@@ -160,3 +160,24 @@ def test_captured_prefill_replays(lens, hip_device):
         ref_o, ref_s = gdn.prefill_run(**t)
         torch.cuda.synchronize()
         assert torch.equal(out, ref_o) and torch.equal(st, ref_s), rnd
+
+
+@pytest.mark.parametrize("lens", [[6], [64], [65, 7]])
+@pytest.mark.parametrize("native", [False, True])
+def test_lazily_cloned_destinations_get_their_own_memory(lens, native, hip_device):
+    """An output and a new state that are lazy clones share memory with their
+    originals until written: the call writes the clones alone."""
+    _announce(f"lazy clones as destinations lens={lens} native={native}")
+    H, HV = 4, 8
+    t = _dev(make_prefill_inputs(lens, H, HV, seed=851), hip_device)
+    ref_o, ref_s = gdn.prefill_run(**t)
+    state, base = t["state"].clone(), torch.zeros_like(t["v"])
+    out, st = torch._lazy_clone(base), torch._lazy_clone(t["state"])
+    if native:
+        assert _host_prefill(t, False, out, st) == 0
+    else:
+        pmod._prefill_checked(t["q"], t["k"], t["v"], t["state"], t["A_log"], t["a"],
+                              t["dt_bias"], t["b"], t["cu_seqlens"], t["scale"], out, st, False)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref_o) and torch.equal(st, ref_s)
+    assert torch.equal(t["state"], state) and not base.any()
