@@ -229,7 +229,17 @@ __device__ __forceinline__ void block_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The same among the lanes of one wave, whose LDS accesses are carried out in
+// Workgroup barrier after this wave's LDS reads and writes (s_waitcnt
+// lgkmcnt(0)) but not its global loads in flight.  The empty asm statements
+// keep the compiler from moving memory accesses across.
+__device__ __forceinline__ void barrier_lds_no_dma() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Ordering among the lanes of one wave, whose LDS accesses are carried out in
 // program order: no instruction, but the fences keep the compiler from moving
 // an access across (the barrier alone is no memory operation, and what one
 // lane stores and another loads looks unrelated in each lane's own view).
@@ -591,7 +601,8 @@ __device__ __forceinline__ f32x4 lds4(const float* ptr) {
 // One chunk's preparation, tokens t0 .. t0 + n - 1 (n: 1..64) of q/k head h,
 // for v-heads hv0 .. hv0 + prep_heads - 1, by the calling wave: the slots go
 // to the workspace (slot c), or with LDS_SLOT (one v-head) to lds_T and
-// lds_scales in the calling workgroup's LDS.
+// lds_scales in the calling workgroup's LDS -- whose other waves' first barrier,
+// that the chunk's rows are in LDS, it joins once its own loads have come.
 template <bool LDS_SLOT>
 __device__ __forceinline__ void prep_chunk(const Params& p, int c, int t0, int n, int hv0, int h,
                                            int prep_heads, PrepLds& lds, uint16_t* lds_T,
@@ -638,6 +649,8 @@ __device__ __forceinline__ void prep_chunk(const Params& p, int c, int t0, int n
         kk[r * (r + 1) / 2 + cb] = acc;
       }
   }
+
+  if constexpr (LDS_SLOT) barrier_lds_no_dma();
 
   // K row scales of the L2-norm (1 when off), |k|^2 from K K^T's diagonal
 #pragma unroll
@@ -910,8 +923,6 @@ void prep_kernel(Params p) {
 // and the buffer's last reads before the second half; the next chunk landed.
 constexpr int kScanWaves = 4;
 constexpr int kScanThreads = 2 * 64 * kScanWaves;
-static_assert(64 * kScanWaves == kThreads, "the one-chunk kernel: main waves only");
-constexpr int kRowDma = kChunk * kDim / 8 / 64;   // DMA instructions per K / Q chunk (16)
 constexpr int kTriDma = 2 * kTriBlocks * kBlk / 8 / 64;   // T diag(beta), hi and lo (12)
 constexpr int kScaleDma = kScaleFloats / 4 / 64;  // row scales (2)
 // K^T operand blocks of a chunk: (key tile t, token block kb), 64 lanes x 8 bf16
@@ -960,16 +971,6 @@ __device__ __forceinline__ unsigned row_bytes(int row, unsigned step, unsigned i
 // Wait for this wave's outstanding vector memory operations (its DMA among
 // them): s_waitcnt vmcnt(0), the other counters left alone.
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
-// Workgroup barrier after this wave's LDS reads and writes (s_waitcnt
-// lgkmcnt(0)) but not its global loads in flight.  The empty asm statements
-// keep the compiler from moving memory accesses across.
-__device__ __forceinline__ void barrier_lds_no_dma() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // Operand label m (0..31) of a 32 x 32 result's row or column as the key (or
 // state column) it stands for: result row 8 q + 4 g + e, register 4 q + e of
@@ -1145,16 +1146,15 @@ __device__ __forceinline__ void p_tile_store(const f32x4& acc, const ScanScales*
   *reinterpret_cast<s16x4*>(dst + kTriBlocks * kBlk) = lo;
 }
 
-// What a chunk's second half needs of its K and Q rows, by wave w (0..3) of
-// four: key tile w of K^T (lane (m, g): tokens 32 R + 8 q + 4 g + e of key
-// 32 w + perm32(m), operand blocks (w, 2 R) and (w, 2 R + 1) of Kt), the
-// wave's three P' tiles, and with the L2-norm 1 / |q_i| of Q rows 16 w .. +
-// 15 into Qn.
+// What a chunk's second half needs of its K and Q rows, share w (0..3) of
+// four.  First what the rows alone give: key tile w of K^T (lane (m, g): tokens
+// 32 R + 8 q + 4 g + e of key 32 w + perm32(m), operand blocks (w, 2 R) and (w,
+// 2 R + 1) of Kt), the products of the share's three P' tiles, and with the
+// L2-norm 1 / |q_i| of Q rows 16 w .. + 15 into Qn.
 template <bool OUT, bool L2>
-__device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
-                                           const ScanScales* __restrict__ Sc,
-                                           uint16_t* Kt, uint16_t* Pb, float* Qn,
-                                           const uint16_t* __restrict__ Sel, int w, int lane) {
+__device__ __forceinline__ void side_products(const ScanIn<OUT>* __restrict__ In, uint16_t* Kt,
+                                              float* Qn, const uint16_t* __restrict__ Sel, int w,
+                                              int lane, f32x4 (&acc)[3]) {
   const int m = lane & 31, g = lane >> 5;
   const unsigned row0 = static_cast<unsigned>(m) * kDim + 8u * (g ^ (m & 15));
 #pragma unroll
@@ -1171,7 +1171,6 @@ __device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
     *reinterpret_cast<s16x8*>(dst + kBlk) = to_bf16x8<1>(kt);
   }
   if constexpr (OUT) {
-    f32x4 acc[3];
 #pragma unroll
     for (int u = 0; u < 3; ++u) {
       acc[u] = f32x4{0, 0, 0, 0};
@@ -1182,8 +1181,6 @@ __device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
         acc[u] = mfma_bf16(ka, qb, acc[u]);
       }
     }
-#pragma unroll
-    for (int u = 0; u < 3; ++u) p_tile_store(acc[u], Sc, PTile(w, u), lane, Pb);
   }
   if constexpr (L2) {
     // four lanes a row (pieces 4 j + lane % 4: the lanes the LDS serves
@@ -1207,6 +1204,16 @@ __device__ __forceinline__ void side_tiles(const ScanIn<OUT>* __restrict__ In,
   }
 }
 
+// Then, with the chunk's scales, the share's P' tiles into Pb.
+template <bool OUT>
+__device__ __forceinline__ void side_store(const ScanScales* Sc, uint16_t* Pb, int w, int lane,
+                                           const f32x4 (&acc)[3]) {
+  if constexpr (OUT) {
+#pragma unroll
+    for (int u = 0; u < 3; ++u) p_tile_store(acc[u], Sc, PTile(w, u), lane, Pb);
+  }
+}
+
 // Chunk ci of a helper wave: the side tiles from In and Sc, then the next
 // chunk's DMA into InN and ScN (their last reads were in the chunk before).
 // The pointers to the chunks' inputs are restrict: the compiler then knows
@@ -1223,7 +1230,9 @@ __device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
                                            const uint16_t* __restrict__ Sel, int ci) {
   const int lane = threadIdx.x & 63;
   const int w = wave_index() - kScanWaves;
-  side_tiles<OUT, L2>(In, Sc, Kt, Pb, Qn, Sel, w, lane);
+  f32x4 acc[3];
+  side_products<OUT, L2>(In, Kt, Qn, Sel, w, lane, acc);
+  side_store<OUT>(Sc, Pb, w, lane, acc);
   if (ci + 1 < cx.nchunks) {                                  // uniform
     // issued while the main waves finish their first half
     const ChunkSrc nsrc = chunk_src(cx, ci + 1);
@@ -1239,9 +1248,11 @@ __device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
 
 // Chunk ci of a main wave, from In and Sc (LAST: the last chunk, which may be
 // a partial one); Kt: the K^T operand blocks; Pb: the P' operand blocks
-// (OUT); Qn: the Q row scales (L2) -- written by the helper waves before the
-// call's first barrier, so not restrict.  OUT: the outputs too (else only the
-// state).  L2: the L2-norm.
+// (OUT); Qn: the Q row scales (L2) -- written by the helper waves within the
+// call, before the barrier ahead of their use, so not restrict; nor are In and
+// Sc, whose slot another wave of the one-chunk kernel (SLOT_LATE) writes until a
+// barrier behind the products that do not need it.  OUT: the outputs too (else
+// only the state).  L2: the L2-norm.
 //
 // The output's intra-chunk term uses P = diag(rq) P' with
 //   P'_ij = scale rk_j e^(gamma_i - gamma_j) (Q K^T)_ij,  j <= i,
@@ -1250,9 +1261,8 @@ __device__ __forceinline__ void help_chunk(const ScanIn<OUT>* __restrict__ In,
 // the 8 items of a lane of P' as the B operand of Delta^T P'^T.  The Q row
 // scales rq = 1 / |q_i| (L2-norm) scale the output row:
 // O = diag(rq) (diag(scale e^gamma) Q S + P' Delta).
-template <bool OUT, bool L2, bool LAST>
-__device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
-                                           const ScanScales* __restrict__ Sc,
+template <bool OUT, bool L2, bool LAST, bool SLOT_LATE = false>
+__device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* In, const ScanScales* Sc,
                                            const uint16_t* Kt, const uint16_t* Pb,
                                            const float* Qn, const ScanCtx& cx,
                                            f32x16 (&st)[4], const uint16_t* __restrict__ Sel,
@@ -1308,6 +1318,8 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* __restrict__ In,
       if constexpr (OUT) o[R] = mfma32_bf16(sl, bq[set][R], o[R]);
     }
   }
+
+  if constexpr (SLOT_LATE) barrier_lds_no_dma();   // the slot is in LDS
 
   // X = V - diag(rk e^gamma) K S, V^T from the selector products; split
   s16x8 xh[4], xl[4];
@@ -1550,6 +1562,24 @@ __device__ __forceinline__ void scan_body(Params p) {
   const int g = lane >> 5;
   const size_t blk = static_cast<size_t>(kDim) * kDim;
 
+  // State registers; k-last storage: 8 consecutive keys are two 16-byte
+  // vectors.
+  f32x16 st[4];
+  const int c = 32 * wave + perm32(m);
+  auto load_st = [&](const float* src) {           // null: zeros
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int key = 32 * t + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
+        const f32x4 v = src != nullptr ? *reinterpret_cast<const f32x4*>(
+                                             src + static_cast<size_t>(c) * kDim + key)
+                                       : f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[t][4 * q + e] = v[e];
+      }
+    }
+  };
   // role: start state, values, where the end state goes
   const float* st_in = nullptr;       // null: zeros (or the identity)
   bool identity = false, values = true, pass_through = false;
@@ -1624,24 +1654,17 @@ __device__ __forceinline__ void scan_body(Params p) {
       seq_slots(s, slot0, nchunks);
   }
 
-  // state registers; k-last storage: 8 consecutive keys are two 16-byte
-  // vectors.  The identity start of a transition gives column c the unit
-  // vector of key c, so that its end column is that start key's column of M.
-  f32x16 st[4];
-  const int c = 32 * wave + perm32(m);
-  const bool load_state = st_in != nullptr && (end > start || pass_through) &&
-                          (FUSE || wave < kScanWaves);   // helper waves hold no columns
+  // The identity start of a transition gives column c the unit vector of key c,
+  // so that its end column is that start key's column of M.
+  load_st(st_in != nullptr && (end > start || pass_through) && wave < kScanWaves
+              ? st_in : nullptr);                  // helper waves hold no columns
+  if constexpr (!OUT) {
+    if (identity) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int key = 32 * t + 16 * (q >> 1) + 8 * g + 4 * (q & 1);
-      const f32x4 v = load_state ? *reinterpret_cast<const f32x4*>(
-                                       st_in + static_cast<size_t>(c) * kDim + key)
-                                 : f32x4{0, 0, 0, 0};
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        st[t][4 * q + e] = identity ? (key + e == c ? 1.0f : 0.0f) : v[e];
+        for (int r = 0; r < 16; ++r)
+          st[t][r] = 32 * t + 16 * (r >> 3) + 8 * g + (r & 7) == c ? 1.0f : 0.0f;
     }
   }
   // selector operands: Sel_h[k][j] = (16 h + k == perm32(j)) over a 16-long k
@@ -1697,20 +1720,36 @@ __device__ __forceinline__ void scan_body(Params p) {
   const ChunkSrc first_src = chunk_src(cx, 0);
   if (wave < 2) *reinterpret_cast<s16x8*>(&Sel[wave * kBlk + lane * 8]) = sel[wave];
   if constexpr (FUSE) {
-    // The chunk's K and Q rows by DMA while this workgroup (four waves, each
-    // main and helper in turn) prepares its slot in LDS, then its one chunk
-    // step.
+    // Main waves bring the chunk's K and Q rows by DMA; helper wave 0 prepares
+    // its slot in LDS, and beside it the other helpers make the K^T and Q K^T
+    // tiles and the main waves their products of the rows and the state.
     static_assert(sizeof(PrepLds) <= sizeof(ScanIn<OUT>), "the preparation fits a buffer");
+    if (wave == kScanWaves) {                                                  // uniform
+      prep_chunk<true>(p, 0, start, end - start, hv, h, 1, *reinterpret_cast<PrepLds*>(&In1),
+                       In0.T, S0.row);             // with the first barrier
+      barrier_lds_no_dma();
+      barrier_lds_no_dma();
+      return;
+    }
+    if (wave > kScanWaves) {                                                   // uniform
+      constexpr int kSide = kScanWaves - 1;        // three waves, share 3 the first one's too
+      const int w = wave - kScanWaves - 1;
+      f32x4 acc[3], acc3[3];
+      barrier_lds_no_dma();
+      side_products<OUT, L2>(&In0, Kt, Qn, Sel, w, lane, acc);
+      if (w == 0) side_products<OUT, L2>(&In0, Kt, Qn, Sel, kSide, lane, acc3);
+      barrier_lds_no_dma();
+      side_store<OUT>(&S0, Pb, w, lane, acc);
+      if (w == 0) side_store<OUT>(&S0, Pb, kSide, lane, acc3);
+      barrier_lds_no_dma();
+      return;
+    }
 #pragma unroll
     for (int part = 0; part < 4; ++part)
       issue_part<OUT, false>(&In0, &S0, cx, first_src, part, wave, lane);
-    if (wave == 0)                                                             // uniform
-      prep_chunk<true>(p, 0, start, end - start, hv, h, 1, *reinterpret_cast<PrepLds*>(&In1),
-                       In0.T, S0.row);
     wait_vmem();
-    block_sync_lds();
-    side_tiles<OUT, L2>(&In0, &S0, Kt, Pb, Qn, Sel, wave, lane);
-    scan_chunk<OUT, L2, true>(&In0, &S0, Kt, Pb, Qn, cx, st, Sel, 0);
+    barrier_lds_no_dma();
+    scan_chunk<OUT, L2, true, true>(&In0, &S0, Kt, Pb, Qn, cx, st, Sel, 0);
     if (st_out != nullptr) store_end(st_out, identity, st, sel);
     return;
   }
@@ -1750,8 +1789,12 @@ void scan_kernel(Params p) {
 
 // Prefills whose tokens all fit one chunk: each (sequence, v-head)
 // workgroup prepares its sequence's chunk in LDS and scans it, in one launch.
+// Its time is a chain: the loads, one wave's preparation, and the chunk step's
+// rest; the step's first half and its tiles run beside the preparation (64
+// tokens in a graph, 4/8 heads 14.2 -> 13.1 us, 16/32 with the L2-norm 14.9 -> 13.4;
+// 13.3 and 14.2 with two workgroups of half a state and four waves preparing).
 template <bool L2>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ __launch_bounds__(kScanThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void one_chunk_kernel(Params p) {
   scan_body<false, false, true, L2, true>(p);
 }
@@ -2162,7 +2205,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, const float
     if (e != hipSuccess) return e;
     p.short_limit = 0;
     auto* fused = p.l2norm ? one_chunk_kernel<true> : one_chunk_kernel<false>;
-    hipLaunchKernelGGL(fused, scan_grid(num_seqs), dim3(kThreads), 0, stream, p);
+    hipLaunchKernelGGL(fused, scan_grid(num_seqs), dim3(kScanThreads), 0, stream, p);
     e = hipGetLastError();
     if (e == hipSuccess) e = mark(3);
     return e;
