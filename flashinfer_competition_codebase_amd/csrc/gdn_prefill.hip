@@ -1016,6 +1016,10 @@ __device__ __forceinline__ f32x16 row_scales(const float* row, int R, int g) {
   return s;
 }
 
+// The Q rows' space where there is one.
+__device__ __forceinline__ uint16_t* state_half(ScanIn<true>& in) { return in.Qr; }
+__device__ __forceinline__ uint16_t* state_half(ScanIn<false>& in) { return in.Kr; }
+
 // The per-workgroup constants of a scan.
 struct ScanCtx {
   const uint16_t* k;
@@ -1466,6 +1470,67 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* In, const ScanScal
   if constexpr (!LAST) barrier_lds_no_dma();   // the next chunk's inputs have landed; this
 }                                              // one's LDS reads are done
 
+// The state between memory and the main waves' registers, through LDS.  A lane's
+// register runs are 16 bytes of a column of its own: straight from or to memory
+// an instruction touches 32 columns, in 64 pieces of 16 bytes.  So the
+// instructions move two whole columns each (512 bytes, 32 lanes), and the layouts
+// are exchanged in 16 KiB of LDS a wave, the 16-byte piece p of column r at
+// position p ^ perm32(r): the lanes that the LDS serves together are on disjoint
+// banks both ways.  Columns 24 .. 31 may lie apart.  Captured calls, GPU time: 4 x
+// 64 tokens at 4/8 heads 17.1 -> 16.2 us (16.4 with two workgroups of half a state
+// each), without a start state 16.0 -> 15.0; 64 x 64 at 16/32 126 -> 115.
+struct StateRows {
+  char* lo;                    // columns 0 .. 23
+  char* hi;                    // columns 24 .. 31
+  __device__ __forceinline__ char* at(int r, int pos) const {
+    return (r < 24 ? lo + r * 512 : hi + (r - 24) * 512) + pos * 16;
+  }
+};
+
+// src, dst: the wave's first column (k-last: 128 consecutive keys a column).
+__device__ __forceinline__ void load_state(f32x16 (&st)[4], const float* src, const StateRows& rows,
+                                           int lane) {
+  const int half = lane >> 5, pos = lane & 31;
+  f32x4 v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    v[i] = *reinterpret_cast<const f32x4*>(src + (2 * i + half) * kDim + 4 * pos);
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    *reinterpret_cast<f32x4*>(rows.at(2 * i + half, pos ^ perm32(2 * i + half))) = v[i];
+  wave_sync_lds();
+  const int m = lane & 31, g = lane >> 5;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 x = *reinterpret_cast<const f32x4*>(
+          rows.at(perm32(m), (8 * t + 4 * (q >> 1) + 2 * g + (q & 1)) ^ m));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) st[t][4 * q + e] = x[e];
+    }
+}
+
+__device__ __forceinline__ void store_state(float* dst, const f32x16 (&st)[4],
+                                            const StateRows& rows) {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));      // as in scan_chunk
+  const int m = lane & 31, g = lane >> 5;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f32x4*>(
+          rows.at(perm32(m), (8 * t + 4 * (q >> 1) + 2 * g + (q & 1)) ^ m)) =
+          f32x4{st[t][4 * q], st[t][4 * q + 1], st[t][4 * q + 2], st[t][4 * q + 3]};
+  wave_sync_lds();
+  const int half = lane >> 5, pos = lane & 31;
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    *reinterpret_cast<f32x4*>(dst + (2 * i + half) * kDim + 4 * pos) =
+        *reinterpret_cast<const f32x4*>(rows.at(2 * i + half, pos ^ perm32(2 * i + half)));
+}
+
 // The end state of a scan: k-last fp32 (element (k, c) at c * 128 + k), or,
 // for a transition M (identity start), as the A operand blocks of the
 // combine's product M S (16x16x32): for row tile t and column block kb, 64
@@ -1656,8 +1721,23 @@ __device__ __forceinline__ void scan_body(Params p) {
 
   // The identity start of a transition gives column c the unit vector of key c,
   // so that its end column is that start key's column of M.
-  load_st(st_in != nullptr && (end > start || pass_through) && wave < kScanWaves
-              ? st_in : nullptr);                  // helper waves hold no columns
+  const float* const src = st_in != nullptr && (end > start || pass_through) && wave < kScanWaves
+                               ? st_in : nullptr;  // helper waves hold no columns
+  if constexpr (OUT && !FUSE) {
+    load_st(nullptr);
+    // LDS that nothing else uses before the scan's first barrier
+    const StateRows rows = {reinterpret_cast<char*>(wave == 0   ? In1.Kr
+                                                    : wave == 1 ? state_half(In1)
+                                                    : wave == 2 ? Kt
+                                                                : In1.T),
+                            reinterpret_cast<char*>(wave == 0   ? In1.Kr + 24 * 256
+                                                    : wave == 1 ? state_half(In1) + 24 * 256
+                                                    : wave == 2 ? Kt + 24 * 256
+                                                                : Pb)};
+    if (src != nullptr) load_state(st, src + 32 * wave * kDim, rows, lane);   // uniform
+  } else {
+    load_st(src);
+  }
   if constexpr (!OUT) {
     if (identity) {
 #pragma unroll
@@ -1717,6 +1797,23 @@ __device__ __forceinline__ void scan_body(Params p) {
   cx.hv = hv;
   cx.values = values;
 
+  // The end state behind the last chunk step, whose middle barrier was the last
+  // use of the K and Q rows.
+  auto store_last = [&]() {
+    if (st_out == nullptr) return;                             // uniform
+    if constexpr (OUT) {
+      uint16_t* const base = wave == 0   ? In0.Kr
+                             : wave == 1 ? In0.Qr
+                             : wave == 2 ? In1.Kr
+                                         : In1.Qr;
+      const StateRows rows = {reinterpret_cast<char*>(base),
+                              reinterpret_cast<char*>(base + 24 * 256)};
+      store_state(st_out + 32 * wave * kDim, st, rows);
+    } else {
+      store_end(st_out, identity, st, sel);
+    }
+  };
+
   const ChunkSrc first_src = chunk_src(cx, 0);
   if (wave < 2) *reinterpret_cast<s16x8*>(&Sel[wave * kBlk + lane * 8]) = sel[wave];
   if constexpr (FUSE) {
@@ -1750,7 +1847,7 @@ __device__ __forceinline__ void scan_body(Params p) {
     wait_vmem();
     barrier_lds_no_dma();
     scan_chunk<OUT, L2, true, true>(&In0, &S0, Kt, Pb, Qn, cx, st, Sel, 0);
-    if (st_out != nullptr) store_end(st_out, identity, st, sel);
+    store_last();
     return;
   }
   if (wave >= kScanWaves) {                                                    // uniform
@@ -1778,7 +1875,7 @@ __device__ __forceinline__ void scan_body(Params p) {
                                Sel, ci);
   scan_chunk<OUT, L2, true>((nchunks & 1) ? &In0 : &In1, (nchunks & 1) ? &S0 : &S1, Kt, Pb, Qn,
                             cx, st, Sel, nchunks - 1);
-  if (st_out != nullptr) store_end(st_out, identity, st, sel);
+  store_last();
 }
 
 template <bool FEW, bool SEG, bool OUT, bool L2>

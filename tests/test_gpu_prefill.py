@@ -740,6 +740,62 @@ def test_preparation_jobs_at_their_edges(lens, H, HV, hip_device):
     _check(t, out, st, loop=False)
 
 
+@pytest.mark.parametrize("limit,lens,longer,H,HV", [
+    # 1024 jobs (a wave each) and 1032 (four waves a workgroup)
+    ("workgroup", [128] * 32 + [192] * 8, [128] * 32 + [192] * 7 + [256], 4, 8),
+    # 4096 (slot, v-head) pairs (a job each) and 4128 (a job a q/k head)
+    ("job", [448] * 16, [448] * 15 + [512], 16, 32),
+])
+def test_preparation_forms_agree_at_their_limits(limit, lens, longer, H, HV, hip_device):
+    """Either side of a limit: against the oracle, and every sequence but the
+    last the same bits."""
+    _announce(f"preparation forms at the {limit} limit H={H} HV={HV}")
+    slots = [(sum(x) + 63) // 64 + len(x) for x in (lens, longer)]
+    jobs = 1024 if limit == "workgroup" else 4096
+    assert slots[0] * HV == jobs and slots[1] == slots[0] + 1
+    L = sum(longer)
+    t = make_prefill_inputs(longer, H, HV, seed=560 + HV)
+    cut = dict(t)
+    short = sum(lens)
+    for n in ("q", "k", "v", "a", "b"):
+        cut[n] = t[n][:short]
+    cut["cu_seqlens"] = t["cu_seqlens"].clone()
+    cut["cu_seqlens"][-1] = short
+    out, st = gdn.prefill_run(**_dev(t, hip_device))
+    out2, st2 = gdn.prefill_run(**_dev(cut, hip_device))
+    torch.cuda.synchronize()
+    assert short == L - 64
+    assert torch.equal(out[:short], out2) and torch.equal(st[:-1], st2[:-1])
+    _check(t, out, st, loop=False)
+
+
+@pytest.mark.parametrize("lens,H,HV", [
+    ([128], 4, 8),                            # one sequence: two chunks
+    ([129], 3, 12),                           # three
+    ([64, 128, 1, 192, 0, 190, 64], 2, 4),    # one, two and three among few
+    ([64] * 70 + [129, 128], 1, 4),           # the offsets kernel
+])
+@pytest.mark.parametrize("l2", [False, True])
+def test_few_chunks_in_both_buffers(lens, H, HV, l2, hip_device):
+    """Plain scans of one, two and three chunks: the buffer that the start state
+    passes through is the second chunk's, and the end state leaves through both."""
+    _announce(f"few chunks lens={lens[:7]} H={H} HV={HV} l2={l2}")
+    t = make_prefill_inputs(lens, H, HV, seed=580 + sum(lens), unit_qk=not l2)
+    td = _dev(t, hip_device)
+    for with_state in (True, False):
+        case = {**t, "state": t["state"] if with_state else None}
+        dev = {**td, "state": td["state"] if with_state else None}
+        out, st = gdn.prefill_run(**dev, use_qk_l2norm=l2)
+        torch.cuda.synchronize()
+        _check(case, out, st, l2=l2)
+        if with_state:                        # in place
+            state, out2 = td["state"].clone(), torch.empty_like(out)
+            gdn.kernel_prefill_hip(**{**td, "state": state}, output=out2, new_state=state,
+                                   use_qk_l2norm=l2)
+            torch.cuda.synchronize()
+            assert torch.equal(out2, out) and torch.equal(state, st)
+
+
 @pytest.mark.parametrize("lens,l2", [([64], False), ([65, 128], True), ([300], True)])
 def test_fast_forgetting_heads_keep_the_split_precision(lens, l2, hip_device):
     """Heads whose log-decay reaches -1000 within a chunk: the state's error
