@@ -896,9 +896,11 @@ __attribute__((amdgpu_waves_per_eu(1, (MULTI && !BF16 && NS == 2) ? 6 : 8))) voi
 // launch takes (B = 1, 32 v-heads: 4 MiB, 0.6 us of traffic in a kernel of
 // 2.5 us, one after another in a graph); together the layers stream like one
 // large batch.  48 layers at B = 1, 16/32 heads (201 MB): 122 us a replay as 48
-// kernels of a graph, 37 us as this one (kernel 31.2 us, 6.5 TB/s).  The layers' pointers are kernel arguments, read
-// by their workgroups through the scalar cache: a captured graph holds them,
-// with no table in device memory to keep.
+// kernels of a graph, 37 us as this one (kernel 31.2 us, 6.5 TB/s).  The layers'
+// pointers are kernel arguments, read by their workgroups through the scalar
+// cache: a captured graph holds them, with no table in device memory to keep.
+// The 4 KiB of arguments hold 51 layers; past kMaxLayers a group takes another
+// launch.
 constexpr int kMaxLayers = 48;
 struct LayerArgs {
   const void* state;

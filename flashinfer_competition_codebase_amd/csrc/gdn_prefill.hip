@@ -25,10 +25,10 @@
 // token with the state in registers, one workgroup per (sequence, v-head,
 // row tile), reading each sequence's token range from cu_seqlens on the
 // device.  Prefills of 57 to 64 tokens in all (every sequence one chunk)
-// whose (sequence, v-head) pairs fill at most half the CUs run one launch of
-// the one-chunk kernel: each workgroup prepares its sequence's chunk in its
-// own LDS (kernel 2's code) and scans it (kernel 3's), so the slot never goes
-// through the workspace.  Larger prefills run the chunkwise kernels -- after
+// with at most 128 (sequence, v-head) pairs run one launch of the one-chunk
+// kernel: each workgroup prepares its sequence's chunk in its own LDS (kernel
+// 2's code) and scans it (kernel 3's), so the slot never goes through the
+// workspace.  Larger prefills run the chunkwise kernels -- after
 // the token kernel's launch, for 2..64 sequences that may all be at most 56
 // tokens long (the host knows only the total): it runs only if every sequence
 // is, and the chunkwise kernels then return at once.
@@ -40,7 +40,7 @@
 //      one sequence, or a few (their slots found in the kernels), it is not
 //      launched.
 //   2. prep, one wave per (chunk slot, q/k head) -- or (chunk slot, v-head)
-//      when all of those fit on the GPU at once: what does not depend on the
+//      when there are few of those: what does not depend on the
 //      state, for all chunks at once -- K K^T (bf16 MFMA: the inputs are bf16,
 //      once per wave), then per v-head the gates and gamma and T by block
 //      recursion (fp32 MFMA) -- into a 14 KiB workspace slot per (chunk,
@@ -103,12 +103,14 @@ constexpr int kDim = 128;            // K == V == 128
 constexpr int kChunk = 64;           // tokens per chunk
 constexpr int kThreads = 256;        // 4 wavefronts
 // Batches whose chunk slots the kernels find themselves, without the offsets
-// kernel: at most kFewSeqs sequences and kFewPrepGroups preparation
-// workgroups (slots x v-heads).  Each workgroup then scans the batch's
-// sequence lengths in one wave, which costs more than the saved launch once
-// there are thousands of them (16 x 512 tokens at 16/32 heads, 4608
-// workgroups: 2% slower; 8 x 1024 at 4/8, 1088: 3% faster; 3 sequences of
-// 30-50 tokens: 18.7 -> 16.3 us).
+// kernel: at most kFewSeqs sequences (one a lane) and kFewPrepGroups (slot,
+// v-head) pairs.  Each preparation wave and scan workgroup then scans the batch's
+// lengths itself, which is always the faster up to there and not always past it
+// (captured calls, in the kernels against the offsets kernel, us: 3 sequences of
+// 40 tokens at 4/8 heads 19.3 / 20.7, 16 x 512 there 49.2 / 51.2, 64 x 128, 1536
+// pairs, 49.4 / 51.1; past it 16 x 1024, 2176 pairs, 74.8 / 77.4, 8 x 1024 at 16/32,
+// 4352, 108.6 / 110.1, but 64 x 64 there, 4096, 126.7 / 124.4 and 64 x 512, 18432, 452.6
+// / 449.5).
 constexpr int kFewSeqs = 64;
 constexpr long long kFewPrepGroups = 2048;
 
@@ -125,12 +127,12 @@ bool few_seqs(long long L, long long N, long long HV) {
   return N > 1 && N <= kFewSeqs && max_slots(L, N) * HV <= kFewPrepGroups;
 }
 // Total tokens up to which the token-by-token kernel runs the prefill (so no
-// sequence is longer).  Measured (one sequence, calls timed from the first to
-// the last event of the timed entry): the token path is 1-3.5 us faster up to
-// 56 tokens at qk4_v8 and qk16_v32, the chunkwise kernels faster from 64.
-// Several short sequences favour the token path far more (4 x 20 tokens: 21.2
-// against 33.5 us at qk4_v8); past the switch the longest sequence is known
-// only on the device (maybe_all_short below).
+// sequence is longer).  The line is where it met the two chunkwise kernels on one
+// sequence; several short ones favour it more (captured calls: 4 x 14 tokens at
+// 4/8 heads 7.7 us, one chunk 12.4).  On one sequence the one-chunk kernel, 12.2 us
+// whatever the tokens, is now faster from 33 tokens at 4/8 heads (56: 19.3 us) and
+// from 25 at 16/32 (56: 25.3 against 12.6): not used there, as the entry points
+// publish the line.
 constexpr int kSmallTokens = 56;
 
 // Batches of 2..kFewSeqs sequences with at most kSmallTokens tokens a
@@ -144,12 +146,16 @@ bool maybe_all_short(long long L, long long N) {
 }
 constexpr float kL2Eps = 1e-6f;
 // A preparation wave takes a whole GVA group of v-heads (K K^T made once for
-// all of them, the v-heads one after another) unless one wave per (slot,
-// v-head) all fit on the GPU at once (16 a CU, 256 CUs): then each takes one
+// all of them, the v-heads one after another) unless there are at most
+// kPrepSplitMaxWaves (slot, v-head) pairs, 16 a CU: then each wave takes one
 // v-head, and the chain of one wave -- the preparation's time on a grid that
-// small -- is one v-head's.
+// small -- is one v-head's.  Twelve waves fit a CU at once, and past them the
+// shorter chain still pays for the second round and for K K^T (captured calls, by
+// v-head against by group, us: 16 x 384 tokens at 16/32 heads, 3584 pairs, 88.5 /
+// 91.9; 4096 pairs: 16 x 448 there 110.3 / 111.2, at 8/32 103.4 / 108.1, 64 x 448 at 4/8
+// 108.2 / 109.7; 16 x 640 at 16/32, 5632 pairs, 147.8 / 143.4).
 constexpr long long kPrepSplitMaxWaves = 4096;
-constexpr long long kPrepSpreadMaxWaves = 1024;     // 4 a CU
+constexpr long long kPrepSpreadMaxWaves = 1024;     // a wave a workgroup up to 4 a CU (kernel 2)
 inline bool prep_split(long long slots, int HV) { return slots * HV <= kPrepSplitMaxWaves; }
 constexpr float kSoftplusThreshold = 20.0f;
 constexpr float kLog2e = 1.44269504088896341f;
@@ -907,8 +913,8 @@ void prep_kernel(Params p) {
 // against eight 16-column waves that each did a share of everything, kernel
 // trace: 64 x 512 tokens at 16/32 heads 429-463 -> 365-405 us, 12 ragged
 // sequences of 7-2048 tokens there 191 -> 152 us, 16 x 1024 at 4/8 76
-// (half-state workgroups on twice the CUs) -> 66 us; ~9.4 k cycles a chunk
-// step.  With all CUs at it the clock falls under the MFMA load (64 x 512: 0.87
+// (two workgroups of half a state each, on twice the CUs) -> 66 us; ~9.4 k cycles a
+// chunk step.  With all CUs at it the clock falls under the MFMA load (64 x 512: 0.87
 // PFLOP/s of bf16 products, where a plain 8192^3 product reaches 1.26).
 //
 // The waves share the chunk's K rows, Q rows and workspace slot, which the
@@ -1017,8 +1023,8 @@ __device__ __forceinline__ f32x16 row_scales(const float* row, int R, int g) {
 }
 
 // The Q rows' space where there is one.
-__device__ __forceinline__ uint16_t* state_half(ScanIn<true>& in) { return in.Qr; }
-__device__ __forceinline__ uint16_t* state_half(ScanIn<false>& in) { return in.Kr; }
+__device__ __forceinline__ uint16_t* q_rows(ScanIn<true>& in) { return in.Qr; }
+__device__ __forceinline__ uint16_t* q_rows(ScanIn<false>& in) { return in.Kr; }
 
 // The per-workgroup constants of a scan.
 struct ScanCtx {
@@ -1346,7 +1352,9 @@ __device__ __forceinline__ void scan_chunk(const ScanIn<OUT>* In, const ScanScal
   // The state's decay of the second half, beside Delta's chains of products
   // (which leave the vector unit idle), where no output accumulators take the
   // registers (first segment launch of 1 x 16384 tokens at 4/8 heads 59.5 ->
-  // 54.6 us; with outputs it spills).
+  // 54.6 us; with outputs it spills).  The segment scan with outputs of a single
+  // sequence spills all the same, 12-16 registers around the loop, and the plain one
+  // behind the offsets kernel with the L2-norm 3.
   const float gl = Sc->row[kRowGl];
   if constexpr (!OUT) {
 #pragma unroll
@@ -1727,11 +1735,11 @@ __device__ __forceinline__ void scan_body(Params p) {
     load_st(nullptr);
     // LDS that nothing else uses before the scan's first barrier
     const StateRows rows = {reinterpret_cast<char*>(wave == 0   ? In1.Kr
-                                                    : wave == 1 ? state_half(In1)
+                                                    : wave == 1 ? q_rows(In1)
                                                     : wave == 2 ? Kt
                                                                 : In1.T),
                             reinterpret_cast<char*>(wave == 0   ? In1.Kr + 24 * 256
-                                                    : wave == 1 ? state_half(In1) + 24 * 256
+                                                    : wave == 1 ? q_rows(In1) + 24 * 256
                                                     : wave == 2 ? Kt + 24 * 256
                                                                 : Pb)};
     if (src != nullptr) load_state(st, src + 32 * wave * kDim, rows, lane);   // uniform
@@ -2024,13 +2032,17 @@ size_t slots_bytes(long long L, long long N, long long HV) {
 // that minimises the estimated critical path, (rounds of the first launch +
 // rounds of the second) x len chunk steps + (nseg - 2) combine steps + the
 // two more launches, with a round of kCUs workgroups and a chunk step
-// costing kStepPerCombine combine steps (measured: ~5.4 us against ~1 us);
-// the batch is cut when that beats its plain scan, (rounds of N HV
-// workgroups) x chunks x kStepPerCombine: from 6 chunks a sequence at N HV
-// = 8 (one 2048-token sequence at qk4_v8: 195 -> ~66 us).  The kernels count
-// each sequence's segments from cu_seqlens (so sequences shorter or longer
-// than the mean get as many as they need), in one wave: at most kFewSeqs
-// sequences.
+// costing kStepPerCombine combine steps; the batch is cut when that beats its
+// plain scan, (rounds of N HV workgroups) x chunks x kStepPerCombine: from 6
+// chunks a sequence at N HV = 8.  A chunk step takes 3.2-3.5 us and a combine step
+// 1.2, a ratio of 3; 5 gives the better lengths (captured calls with 5 / 3 / no
+// segments, us: 2048 tokens at 4/8 heads 56.2 / 57.2 / 116.6, 16384 there 145.4 /
+// 150.1 / 841.5, 8192 at 16/32 213.1 / 218.6 / 454.0) but cuts sequences of 6 and 7
+// chunks, and some batches, that the plain scan takes faster (384 tokens at 4/8
+// 36.2 / 31.5 / 31.5, 448 36.7 / 34.9 / 34.8, 4 x 448 46.4 / 37.0 / 36.6, 8 x 1024 87.5 /
+// 87.0 / 73.7; from 512 tokens on one sequence gains by it).  The kernels count each sequence's
+// segments from cu_seqlens (so sequences shorter or longer than the mean get as
+// many as they need), in one wave: at most kFewSeqs sequences.
 constexpr long long kSegMaxHeads = 256;  // N HV workgroups that fill the GPU unsegmented
 constexpr long long kSegMinLen = 2;
 constexpr long long kCUs = 256;
@@ -2056,10 +2068,12 @@ SegPlan seg_plan(long long L, long long N, long long HV) {
 }
 
 // Prefills past the token path whose tokens all fit one chunk (so every
-// sequence is one chunk) and whose workgroups fill at most half the CUs: one
-// launch in which each (sequence, v-head) workgroup prepares its chunk in LDS
-// and scans it -- no workspace round trip and one launch instead of the
-// preparation's and the scan's.
+// sequence is one chunk), with at most 128 (sequence, v-head) workgroups: one
+// launch in which each prepares its chunk in LDS and scans it -- no workspace
+// round trip and one launch instead of two or three (captured calls against
+// those: 64 tokens at 4/8 heads 12.3 / 14.9 us, 4 x 16 at 16/32 13.3 / 22.1).  Past 128
+// it depends on the lengths, which the host does not know: 5 x 12 tokens at 16/32
+// 14.0 / 21.0 us, but 30 x 2 at 4/8, which the token kernel takes, 15.3 / 13.9.
 bool fused_prefill(long long L, long long N, long long HV) {
   return L > kSmallTokens && L <= kChunk && N >= 1 && 2 * N * HV <= kCUs;
 }

@@ -59,7 +59,7 @@ def _check(t, out, st, l2=False, loop=True):
 @pytest.mark.parametrize("seqlens,H,HV", [
     ([70] + [1] * 63, 4, 8),          # 64 sequences: chunk slots found in the kernels
     ([70] + [1] * 64, 4, 8),          # 65: the chunk-offsets scan
-    ([70] + [1] * 99, 1, 1),          # 100: the offsets scan, then half-state scan workgroups
+    ([70] + [1] * 99, 1, 1),          # 100 of one head: the offsets scan
     ([0, 130, 0, 0, 64, 1, 0], 2, 4), # empty sequences among few
     ([6], 4, 8),                      # the size of the reference's prefill workload 0
     ([1], 4, 8),
@@ -709,9 +709,9 @@ def test_one_chunk_kernel(seqlens, H, HV, l2, with_state, hip_device):
 @pytest.mark.parametrize("l2", [False, True])
 def test_one_chunk_kernel_matches_the_chunkwise_kernels_bitwise(l2, hip_device):
     """A 64-token sequence alone (the one-chunk kernel) and first in a batch
-    of 64 + 65 tokens (the preparation kernel, one v-head a workgroup, and
-    the half-state scan): the same bits, since the one-chunk kernel runs
-    those kernels' arithmetic with the slot kept in LDS."""
+    of 64 + 65 tokens (the preparation kernel, a v-head a wave, and the
+    scan): the same bits, since the one-chunk kernel runs those kernels'
+    arithmetic with the slot kept in LDS."""
     _announce(f"one-chunk kernel vs chunkwise kernels, bitwise, l2={l2}")
     t = make_prefill_inputs([64, 65], 4, 8, seed=71)
     assert gdn.prefill.prefill_dispatches(129, 2, 8) == 2

@@ -67,8 +67,8 @@ def test_workspace_size_formula():
         offsets = 0 if N == 1 or (N <= 64 and chunks * HV <= 2048) else 1
         # 2..64 sequences of at most 56 tokens on average: the token kernel first
         token = 1 if 2 <= N <= 64 and 56 < L <= 56 * N else 0
-        # at most one chunk in all, half-state workgroups on at most all CUs:
-        # the one-chunk kernel alone
+        # at most one chunk in all and at most 128 (sequence, v-head) pairs: the
+        # one-chunk kernel alone
         one_chunk = 56 < L <= 64 and 2 * N * HV <= 256
         assert lib.gdn_prefill_dispatches(L, N, HV) == (
             0 if N == 0 else 1 if (L <= 56 and N <= 65535) or one_chunk else
