@@ -5,7 +5,7 @@
 // us, and the Python checks of its twelve tensors, the workspace, the stream
 // and the 22-argument ctypes call made it 20.3 us a call; a value-returning
 // decode step of a few heads took 16.1.  These functions make the same checks,
-// allocations and call: 5.5 and 6.2 us.  They are a fast path only: arguments
+// allocations and call: 5.5-6.4 and 6.2 us.  They are a fast path only: arguments
 // outside what they accept (anything the Python path would refuse, convert or
 // treat specially) return None, nothing done, and the Python path takes the
 // call from the start, so its errors and conversions stay as they are.
